@@ -52,8 +52,8 @@ def parse_args():
                          "backward) and the step reads them from HBM; recompute = the step projects X and G "
                          "again (two extra passes over the narrower of each pair)")
     ap.add_argument("--stream-factors", choices=["on", "off"], default="on",
-                    help="c3: on = factor rows whose leaves each take a 16-row block of the plane (rank <= 16, "
-                         "up to three blocks) stream P through LDS (odp_seg_factor_stream); off = the "
+                    help="c3: on = factor rows whose leaves each take 16-row blocks of the plane of their own "
+                         "stream P through LDS (odp_seg_factor_stream_tables); off = the "
                          "register-staged odp_seg_factor tiles (bit-identical results)")
     ap.add_argument("--seed", type=int, default=0)
     ap.add_argument("--linear-pe-gb", type=float, default=None,
@@ -102,8 +102,9 @@ def kernel_label(stage, key):
         return {"sqnorm": "k_sqnorm", "scale_sum": "k_scale_sum", "nonfinite": "k_nonfinite_cols",
                 "pack": "k_pack_factors", "planes": "k_pack_planes",
                 "factor_project": "k_factor_project_bf16"}[stage]
-    if stage == "factor_stream":  # keyed by rank blocks
-        return f"k_factor_stream_bf16<{key}>"
+    if stage in ("factor_stream", "factor_stream_long"):
+        # One launch over the tables of several rank block counts; one table alone names its count.
+        return "k_factor_stream_bf16" if isinstance(key, tuple) else f"k_factor_stream_bf16<{key}>"
     dt, nkb = key
     base = {"project": "k_project_stream", "factor": "k_factor"}[stage]
     if dt == torch.bfloat16:

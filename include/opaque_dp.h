@@ -18,7 +18,7 @@
  * replace the following internals of its DP-SGD hot path
  * (paths relative to packages/):
  *   odp_project or odp_pack_planes, odp_seg_factor_project, odp_seg_factor,
- *   odp_seg_factor_stream         -> per-sample LoRA factor gradients,
+ *   odp_seg_factor_stream(_tables) -> per-sample LoRA factor gradients,
  *       opaque-patches/src/opaque/api/patches/kernels/lora.py:164-176
  *       (dA[i] = s X[i]^T (G[i] B^T), dB[i] = s (X[i] A)^T G[i]) and the
  *       per-example squared norms of clip_pytree,
@@ -250,6 +250,23 @@ int odp_seg_factor_stream(odp_stream_t stream, const int64_t* problems,
                           const int32_t* work_start, int32_t n_prob, int32_t total_blocks,
                           const int32_t* seg_row_start, const int32_t* seg_row_len,
                           const int32_t* seg_example, double* part, int64_t part_stride, int32_t nkb);
+
+/* ---- odp_seg_factor_stream_tables: streamed tables in one launch --------
+ * odp_seg_factor_stream over up to four tables at once: problems[k],
+ * block_map[k], n_prob[k], total_blocks[k] (host arrays of four; a missing
+ * table has n_prob 0) are the problems with k + 1 rank blocks.  Instead of
+ * work_start a table has a device array of total_blocks (row, workgroup of
+ * the row) int32 pairs, in launch order: workgroup w of a row takes column
+ * group w % ODP_FT_GROUPS of its segment w / ODP_FT_GROUPS.  Every leaf
+ * starts at a column of Q that is a multiple of 16; a leaf of rank above 16
+ * takes the blocks that follow (rank <= 64).  Segments may have any length
+ * whose rows span less than 2 GiB of P.  Rows, squares and partial slots as
+ * odp_seg_factor's with the same rank blocks, bit for bit.               */
+int odp_seg_factor_stream_tables(odp_stream_t stream, const int64_t* const* problems,
+                                 const int32_t* const* block_map, const int32_t* n_prob,
+                                 const int32_t* total_blocks, const int32_t* seg_row_start,
+                                 const int32_t* seg_row_len, const int32_t* seg_example, double* part,
+                                 int64_t part_stride);
 
 /* ---- odp_sqnorm: squared norms of materialised per-example tensors -------
  * For leaves that are not behind a captured linear op, the per-example

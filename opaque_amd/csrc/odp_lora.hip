@@ -486,38 +486,42 @@ __host__ __device__ constexpr int fs_groups(int nchunks) {
   return nchunks <= 0 ? 1 : (nchunks + ODP_FS_GROUP - 1) / ODP_FS_GROUP;
 }
 
+// LDS elements of one stage of the pass: a P tile and NKB 16-row blocks of
+// Q.  Q rows are 64 tokens = 128 bytes, unpadded, with 16-byte slot q of row
+// t at slot q ^ (t & 7) (16 rows read at one slot without bank conflicts):
+// four rank blocks then make a stage of exactly 40 KB, so that two
+// workgroups of two stages fill the CU's 160 KB.
+__host__ __device__ constexpr int fp_stage(int nkb) { return FP_T * FP_MT + 16 * nkb * FP_T; }
+
 // One pass over P = G of a segment in 256-column chunks.  PROJ: the fused
 // G side above (dB rows and U = G B^T, one workgroup per segment, all
 // chunks).  !PROJ: the planes are given, so the pass forms only the
 // per-example factor rows pe[k][m] = scaling * sum_t Q[k][t] P[t][m] (dB
 // from G and V, or dA from X and U) of a problem with NKB 16-row blocks of
-// Q, each holding at most one leaf that starts at the block (rank <= 16):
-// the pipeline of the fused kernel without B, U and its registers.  A
-// workgroup then takes one of the row's ODP_FT_GROUPS groups of
-// consecutive chunks of its segment.  Both compute each chunk's rows,
-// squares and partial slots exactly as k_factor_bf16<NKB> does for its
-// 256-column tile (same token blocks, same order).
+// Q, whose leaves each start at a block (a leaf of rank above 16 spans the
+// blocks that follow): the pipeline of the fused kernel without B, U and its
+// registers.  A workgroup then takes one of the row's ODP_FT_GROUPS groups
+// of consecutive chunks of its segment, whose length only `max_steps`
+// bounds.  Both compute each chunk's rows, squares and partial slots exactly
+// as k_factor_bf16<NKB> does for its 256-column tile (same token blocks,
+// same order).
 template <bool PROJ, int NKB>
-__device__ __forceinline__ void factor_pass_bf16(const int64_t* __restrict__ probs, const int32_t* __restrict__ ws,
-                                                 int n_prob, const int32_t* __restrict__ sstart,
+__device__ __forceinline__ void factor_pass_bf16(const int64_t* __restrict__ f, int local, int max_steps,
+                                                 uint16_t* lds, const int32_t* __restrict__ sstart,
                                                  const int32_t* __restrict__ slen, const int32_t* __restrict__ sex,
                                                  double* __restrict__ part, int64_t part_stride) {
-  static_assert(NKB >= 1 && NKB <= 3 && (!PROJ || NKB == 1), "one to three rank blocks; the fused G side has one");
+  static_assert(NKB >= 1 && NKB <= 4 && (!PROJ || NKB == 1), "one to four rank blocks; the fused G side has one");
   constexpr int NJ = FP_MT / 64, PP = FP_MT;  // unpadded, XOR-swizzled G rows
-  constexpr int QP = lds_pitch(FP_T), QROWS = 16 * NKB;
-  constexpr int PTILE = FP_T * PP, STAGE = PTILE + QROWS * QP;
+  constexpr int QROWS = 16 * NKB;
+  constexpr int PTILE = FP_T * PP, STAGE = fp_stage(NKB);
   constexpr int QPC = FP_T / 8;                  // V pieces per row per step
   constexpr int NQP = QPC * QROWS;               // V pieces per step: 128 per rank block
   constexpr int NQ = (NQP + 255) / 256;          // per thread (waves past NQP issue none)
   static_assert(NQP % 128 == 0, "V pieces cover whole waves");
-  // Stores a chunk's flush issues (every one unconditional): NJ rows and a
-  // partial per rank block.  The step-1 wait below encodes it in 4 bits.
+  // Stores a chunk's rows issue (every one unconditional): NJ rows and a
+  // partial per rank block.  The step-1 wait below encodes it in 6 bits.
   constexpr int NFLUSH = NKB * (NJ + 1);
-  static_assert(NFLUSH <= 15, "vmcnt immediate");
-  __shared__ __attribute__((aligned(16))) uint16_t lds[2 * STAGE];
-  const int bid = blockIdx.x;
-  const int p = odp_find_problem(ws, n_prob, bid);
-  const int64_t* f = probs + (int64_t)p * ODP_FT_FIELDS;
+  static_assert(NFLUSH < 64, "vmcnt immediate");
   const uint16_t* P = (const uint16_t*)f[ODP_FT_P];
   const int32_t ldp = (int32_t)f[ODP_FT_LDP], M = (int32_t)f[ODP_FT_M];
   const int32_t ldq = (int32_t)f[ODP_FT_LDQ];
@@ -526,18 +530,17 @@ __device__ __forceinline__ void factor_pass_bf16(const int64_t* __restrict__ pro
   const uint16_t* W = PROJ ? (const uint16_t*)f[ODP_FP_W] : nullptr;
 
   const int nchunks = (M + FP_MT - 1) / FP_MT;
-  const int local = bid - ws[p];
   int seg, c_begin, c_end;
   if constexpr (PROJ) {
     seg = local;
     c_begin = 0;
     c_end = nchunks;
   } else {
-    const int64_t ng = f[ODP_FT_GROUPS] > 0 ? f[ODP_FT_GROUPS] : 1;
-    seg = (int)(local / ng);
-    const int64_t grp = local - seg * ng;
-    c_begin = (int)(grp * nchunks / ng);
-    c_end = (int)((grp + 1) * nchunks / ng);
+    const int ng = f[ODP_FT_GROUPS] > 0 ? (int)f[ODP_FT_GROUPS] : 1;
+    seg = local / ng;
+    const int grp = local - seg * ng;
+    c_begin = (int)((uint32_t)grp * (uint32_t)nchunks / (uint32_t)ng);
+    c_end = (int)((uint32_t)(grp + 1) * (uint32_t)nchunks / (uint32_t)ng);
     // Workgroups past the row's segments (a table whose work_start counts
     // more than n_seg * groups) have nothing to do.
     if (seg >= (int)f[ODP_FT_NSEG]) return;
@@ -547,8 +550,7 @@ __device__ __forceinline__ void factor_pass_bf16(const int64_t* __restrict__ pro
   const int ex = sex[gs];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int32_t t_lo = rs & ~7;
-  int nsteps = len > 0 ? (t_hi - t_lo + FP_T - 1) / FP_T : 0;
-  nsteps = nsteps < FP_STEPS ? nsteps : FP_STEPS;  // the host keeps segments within bounds
+  const int nsteps = len > 0 ? (t_hi - t_lo + FP_T - 1) / FP_T : 0;
 
   // G through a buffer resource over the segment's rows, loaded straight
   // into LDS: rows outside the segment (offsets below it wrap past the end)
@@ -572,7 +574,7 @@ __device__ __forceinline__ void factor_pass_bf16(const int64_t* __restrict__ pro
     vown[i] = __builtin_amdgcn_readfirstlane(wave) * 64 + 256 * i < NQP;
     const int qrow = ((tid + 256 * i) % NQP) / QPC;
     qsrc[i] = (const uint16_t*)f[ODP_FT_Q] + (int64_t)qrow * ldq;
-    qdst_base[i] = lds + PTILE + qrow * QP + 8 * qpc;
+    qdst_base[i] = lds + PTILE + qrow * FP_T + 8 * (qpc ^ (qrow & 7));
   }
 
   auto load = [&](uint16_t* stage, int32_t t0, int32_t m_base, u32x4_t (&qv)[NQ]) {
@@ -612,128 +614,111 @@ __device__ __forceinline__ void factor_pass_bf16(const int64_t* __restrict__ pro
   f32x4_t acc_u[PROJ ? FP_STEPS : 1];
 #pragma unroll
   for (int st = 0; st < (PROJ ? FP_STEPS : 1); ++st) acc_u[st] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  // The leaf of each rank block (bf16 rows): the one that starts at column
-  // 16 kb of Q, if any (rank 0 otherwise: nothing stored, no partial).
+  // The leaf of each rank block (bf16 rows): the one whose columns of Q hold
+  // the block, if any (rank 0 otherwise: nothing stored, no partial).  lpe
+  // points at the block's first row of this segment; a leaf's blocks share
+  // one partial slot, written with its last block.
   const FactorLeaves L = read_leaves(f);
   uint16_t* lpe[NKB];
-  int lrank[NKB];
+  int lrank[NKB];        // rows of the leaf in this block
   int64_t lslot[NKB];
+  bool lcont[NKB], llast[NKB];  // the block continues the leaf above it / ends its leaf
 #pragma unroll
   for (int kb = 0; kb < NKB; ++kb) {
     lpe[kb] = nullptr;
     lrank[kb] = 0;
     lslot[kb] = 0;
+    lcont[kb] = llast[kb] = false;
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (q < L.n && L.col0[q] == 16 * kb) {
-        lpe[kb] = (uint16_t*)L.pe[q];
-        lrank[kb] = L.rank[q] < 16 ? L.rank[q] : 16;
+    for (int q = 0; q < 4; ++q) {
+      const int k0 = 16 * kb - L.col0[q];  // the block's first row within leaf q
+      if (q < L.n && k0 >= 0 && k0 < L.rank[q]) {
+        lpe[kb] = (uint16_t*)L.pe[q] + ((int64_t)seg * L.rank[q] + k0) * M;
+        lrank[kb] = L.rank[q] - k0 < 16 ? L.rank[q] - k0 : 16;
         lslot[kb] = L.slot[q];
+        lcont[kb] = k0 > 0;
+        llast[kb] = k0 + 16 >= L.rank[q];
       }
+    }
   }
-  // A segment longer than FP_STEPS steps does not fit this pass (the host
+  // A segment longer than max_steps steps does not fit this pass (the host
   // keeps segments within odp_factor_project_max_len()): its partial slots
   // become NaN, so that its norm and clip factor show it, and nothing else
   // is written.
-  if (len > 0 && (t_hi - t_lo + FP_T - 1) / FP_T > FP_STEPS) {
+  if (nsteps > max_steps) {
     if (lane == 0)
       for (int kb = 0; kb < NKB; ++kb)
-        if (lrank[kb] > 0)
+        if (llast[kb])
           for (int c = c_begin; c < c_end; ++c)
             odp_gstore(part + (int64_t)ex * part_stride + lslot[kb] + ODP_FT_WAVE_SLOTS * c + wave,
                        __builtin_nan(""));
     return;
   }
 
-  // A chunk's rows (bf16) and this wave's norm partials wait in registers
-  // and are stored after the next step's barrier: a barrier waits for every
-  // memory operation in flight, so stores issued just before one would
-  // stall it for their whole latency.  The arithmetic is factor_epilogue's
-  // for one leaf per rank block, in the same order.
-  uint32_t pend[NKB][NJ * 2];
-  double pend_sq[NKB];
-  int32_t pend_m0 = -1, pend_tile = 0;  // pend_m0 < 0: nothing pending
-  auto hold = [&](const f32x4_t (&acc)[NJ][NKB], int32_t m_base, int tile) {
+  // A chunk's rows (bf16) and this wave's norm partials are formed and
+  // stored in step 0 of the next chunk, after that step has issued the loads
+  // of step 1: a barrier waits for every memory operation in flight, so
+  // stores issued just before one would stall it for their whole latency,
+  // and the arithmetic (about 1500 cycles per rank block) would delay the
+  // next loads.  The arithmetic is factor_epilogue's, in the same order.
+  //
+  // Each 16 x 16 block of rows leaves as 8-byte pieces: a 4 x 4 transpose
+  // within each quad of lanes (two exchanges) turns lane (g, 4q + t)'s
+  // column of rows 4g .. 4g + 3 into row 4g + t, columns 4q .. 4q + 3.  The
+  // stores are buffer stores issued unconditionally (an offset past the end
+  // drops a store with nothing to write, as all of them before the first
+  // chunk): the compiler then knows that exactly NFLUSH of them follow B's
+  // loads, and the MFMAs that wait for B do not wait for the stores.
+  auto emit = [&](const f32x4_t (&acc)[NJ][NKB], bool live, int32_t m_base, int tile) __attribute__((always_inline)) {
+    const int t = lane & 3, tl = t & 1, th = t >> 1;
+    const int kt = 4 * (lane >> 4) + t;
+    double wsum = 0.0;
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb) {
       const int rk = lrank[kb];
-      double wsum = 0.0, cs[4];
+      const __amdgpu_buffer_rsrc_t pe_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)lpe[kb], (short)0, (int)((uint32_t)rk * (uint32_t)M * 2u), ODP_BUFFER_DWORD3);
+      const __amdgpu_buffer_rsrc_t part_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(part + (int64_t)ex * part_stride + lslot[kb]), (short)0,
+          llast[kb] ? (int)(ODP_FT_WAVE_SLOTS * (uint32_t)nchunks * 8u) : 0, ODP_BUFFER_DWORD3);
+      double cs[4] = {0.0, 0.0, 0.0, 0.0};
+      if (!lcont[kb]) wsum = 0.0;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        cs[i] = 0.0;
-        const int k = 4 * (lane >> 4) + i;
+      for (int j = 0; j < NJ; ++j) {
+        const int32_t m = m_base + (NJ * wave + j) * 16 + (lane & 15);
+        uint32_t h[4];
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          const int32_t m = m_base + (NJ * wave + j) * 16 + (lane & 15);
-          const float v = scale * acc[j][kb][i];
-          const uint32_t h = odp_f2bf(v);
-          if (i & 1)
-            pend[kb][2 * j + (i >> 1)] |= h << 16;
-          else
-            pend[kb][2 * j + (i >> 1)] = h;
-          if (k < rk && m < M) {
-            const float vq = odp_bf2f((uint16_t)h);  // the value as stored
+        for (int i = 0; i < 4; ++i) {
+          h[i] = odp_f2bf(scale * acc[j][kb][i]);
+          if (4 * (lane >> 4) + i < rk && m < M) {
+            const float vq = odp_bf2f((uint16_t)h[i]);  // the value as stored
             const float vf = isfinite(vq) ? vq : 0.f;
             cs[i] += (double)__fmul_rn(vf, vf);
           }
         }
+        // Rows of the other parity to the odd/even neighbour.
+        const uint32_t r1 = quad_x1(tl ? (h[0] | (h[2] << 16)) : (h[1] | (h[3] << 16)));
+        // Rows 4g + 2a + tl, columns of this lane pair (low half: even column).
+        const uint32_t p0 = tl ? ((r1 & 0xffffu) | (h[1] << 16)) : (h[0] | (r1 << 16));
+        const uint32_t p1 = tl ? ((r1 >> 16) | (h[3] << 16)) : (h[2] | (r1 & 0xffff0000u));
+        // Row pairs across the two lane pairs of the quad.
+        const uint32_t r2 = quad_x2(th ? p0 : p1);
+        const uint32_t keep = th ? p1 : p0;
+        const int32_t mq = m_base + (NJ * wave + j) * 16 + 4 * ((lane & 15) >> 2);
+        const uint32_t off = live && kt < rk && mq < M ? ((uint32_t)kt * (uint32_t)M + (uint32_t)mq) * 2u : 0x80000000u;
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{th ? r2 : keep, th ? keep : r2}, pe_rsrc, (int)off, 0, 0);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const double v = row_sum16(cs[i]);
         if (4 * (lane >> 4) + i < rk) wsum += v;
       }
-      pend_sq[kb] = rows_sum4(wsum);
-    }
-    pend_m0 = m_base;
-    pend_tile = tile;
-  };
-  // Each 16 x 16 block of rows leaves as 8-byte pieces: a 4 x 4 transpose
-  // within each quad of lanes (two exchanges) turns lane (g, 4q + t)'s
-  // column of rows 4g .. 4g + 3 into row 4g + t, columns 4q .. 4q + 3.  The
-  // stores are buffer stores issued unconditionally (an offset past the end
-  // drops a store with nothing to write): the compiler then knows that
-  // exactly NFLUSH of them follow B's loads, and the MFMAs that wait for B
-  // do not wait for the stores.
-  __amdgpu_buffer_rsrc_t pe_rsrc[NKB], part_rsrc[NKB];
-#pragma unroll
-  for (int kb = 0; kb < NKB; ++kb) {
-    pe_rsrc[kb] = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(lpe[kb] + (int64_t)seg * lrank[kb] * M), (short)0,
-        (int)((uint32_t)lrank[kb] * (uint32_t)M * 2u), ODP_BUFFER_DWORD3);
-    part_rsrc[kb] = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(part + (int64_t)ex * part_stride + lslot[kb]), (short)0,
-        lrank[kb] > 0 ? (int)(ODP_FT_WAVE_SLOTS * (uint32_t)nchunks * 8u) : 0, ODP_BUFFER_DWORD3);
-  }
-  auto flush = [&]() {
-    const bool live = pend_m0 >= 0;
-    const int t = lane & 3, tl = t & 1, th = t >> 1;
-    const int k = 4 * (lane >> 4) + t;
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb) {
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const uint32_t h0 = pend[kb][2 * j] & 0xffffu, h1 = pend[kb][2 * j] >> 16;
-        const uint32_t h2 = pend[kb][2 * j + 1] & 0xffffu, h3 = pend[kb][2 * j + 1] >> 16;
-        // Rows of the other parity to the odd/even neighbour.
-        const uint32_t r1 = quad_x1(tl ? (h0 | (h2 << 16)) : (h1 | (h3 << 16)));
-        // Rows 4g + 2a + tl, columns of this lane pair (low half: even column).
-        const uint32_t p0 = tl ? ((r1 & 0xffffu) | (h1 << 16)) : (h0 | (r1 << 16));
-        const uint32_t p1 = tl ? ((r1 >> 16) | (h3 << 16)) : (h2 | (r1 & 0xffff0000u));
-        // Row pairs across the two lane pairs of the quad.
-        const uint32_t r2 = quad_x2(th ? p0 : p1);
-        const uint32_t keep = th ? p1 : p0;
-        const int32_t m = pend_m0 + (NJ * wave + j) * 16 + 4 * ((lane & 15) >> 2);
-        const uint32_t off =
-            live && k < lrank[kb] && m < M ? ((uint32_t)k * (uint32_t)M + (uint32_t)m) * 2u : 0x80000000u;
-        __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{th ? r2 : keep, th ? keep : r2}, pe_rsrc[kb], (int)off, 0, 0);
-      }
+      const double sq = rows_sum4(wsum);
       const uint32_t poff =
-          live && lane == 0 ? (uint32_t)(ODP_FT_WAVE_SLOTS * pend_tile + wave) * 8u : 0x80000000u;
-      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, pend_sq[kb]), part_rsrc[kb], (int)poff, 0,
-                                            0);
+          live && lane == 0 ? (uint32_t)(ODP_FT_WAVE_SLOTS * tile + wave) * 8u : 0x80000000u;
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, sq), part_rsrc, (int)poff, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);  // one rank block's temporaries at a time
     }
-    pend_m0 = -1;
   };
   // B's chunk as MFMA B operands: k-step ks covers columns 32 ks .. + 31,
   // lane holds B[lane & 15][32 ks + 8 (lane >> 4) .. + 7].  Loaded after the
@@ -745,6 +730,14 @@ __device__ __forceinline__ void factor_pass_bf16(const int64_t* __restrict__ pro
   const uint32_t wrow = (lane & 15) < r ? (uint32_t)(lane & 15) * (uint32_t)M : 0x40000000u;
 
   u32x4_t qv[NQ];
+  f32x4_t acc[NJ][NKB];
+  auto zero = [&]() {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb) acc[j][kb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  };
+  zero();
   int buf = 0;
   if (nsteps > 0 && c_begin < c_end) load(lds, t_lo, c_begin * FP_MT, qv);
   for (int c = c_begin; c < c_end; ++c) {
@@ -755,24 +748,19 @@ __device__ __forceinline__ void factor_pass_bf16(const int64_t* __restrict__ pro
     int32_t tc0 = t_lo;
     __asm__ volatile("" : "+s"(tc0));
     bf16x8_t wf[FP_MT / 32];
-    f32x4_t acc[NJ][NKB];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) acc[j][kb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
     // One step: the next stage's loads go into `nxt` while the step reads
     // `sp`.  The two are restrict-qualified, so the compiler's scoped alias
     // information tells them apart and the transposing reads of `sp` do
     // not wait for the loads just issued into `nxt` (a barrier at the top
     // of each step already waits for the stage's own loads).
-    auto step = [&](uint16_t* __restrict__ nxt, const uint16_t* __restrict__ sp,
-                    int st) __attribute__((always_inline)) {
+    auto step = [&](uint16_t* __restrict__ nxt, const uint16_t* __restrict__ sp, int st,
+                    bool first) __attribute__((always_inline)) {
       if (st + 1 < nsteps)
         load(nxt, tc0 + (st + 1) * FP_T, m_base, qv);
       else if (c + 1 < c_end)
         load(nxt, tc0, m_base + FP_MT, qv);
-      if (st == 0) {
+      if (first) {
         if constexpr (PROJ) {
           // B's loads before the stores: the MFMAs that wait for B then do
           // not wait for the stores too (memory operations complete in
@@ -785,16 +773,18 @@ __device__ __forceinline__ void factor_pass_bf16(const int64_t* __restrict__ pro
           }
         }
         __builtin_amdgcn_sched_barrier(0);
-        flush();
+        emit(acc, c > c_begin, m_base - FP_MT, c - 1);
+        zero();
       }
       __builtin_amdgcn_sched_barrier(0);  // keep the prefetch ahead of the compute
       // Factor rows: B operand = P columns by transposing reads, A = Q.
 #pragma unroll
       for (int u = 0; u < FP_T / 32; ++u) {
-        const int tc = 32 * u + 8 * (lane >> 4);
+        const int qs = (4 * u + (lane >> 4)) ^ (lane & 7);  // slot of the lane's 8 tokens
         u32x4_t vv[NKB];
 #pragma unroll
-        for (int kb = 0; kb < NKB; ++kb) vv[kb] = *(const u32x4_t*)&sp[PTILE + (16 * kb + (lane & 15)) * QP + tc];
+        for (int kb = 0; kb < NKB; ++kb)
+          vv[kb] = *(const u32x4_t*)&sp[PTILE + (16 * kb + (lane & 15)) * FP_T + 8 * qs];
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
           const int m0 = (NJ * wave + j) * 16, cc = lane & 15;
@@ -822,36 +812,48 @@ __device__ __forceinline__ void factor_pass_bf16(const int64_t* __restrict__ pro
         }
       }
     };
-    // Steps as nested conditionals (step st + 1 inside step st): each step
-    // is then reached only from the one before it, and the compiler counts
-    // the memory operations in flight exactly across them.
+    // A step's loads (this wave's) must have landed and its V pieces be
+    // written before the barrier.  Vector memory operations complete in
+    // issue order as s_waitcnt counts them, and step 0 issues the stage's
+    // loads before B's loads and the NFLUSH stores of the previous chunk: at
+    // step 1, vmcnt <= NFLUSH covers the stage while the stores drain.
+    // Other steps wait for everything.
+    auto one = [&](int st, auto K) __attribute__((always_inline)) {
+      constexpr int kind = decltype(K)::value < 2 ? decltype(K)::value : 2;  // step 0, step 1, a later one
+      store_q(buf, tc0 + st * FP_T, qv);
+      if (kind == 1)
+        __builtin_amdgcn_s_waitcnt(0x0070 | (NFLUSH & 15) | ((NFLUSH >> 4) << 14));  // vmcnt(NFLUSH) lgkmcnt(0)
+      else
+        __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+      __asm__ volatile("s_barrier" ::: "memory");
+      step(lds + (buf ^ 1) * STAGE, lds + buf * STAGE, st, kind == 0);
+      buf ^= 1;
+    };
+    // Steps 0 and 1 by themselves, each reached only from the one before it,
+    // so that the compiler counts the memory operations in flight exactly
+    // across them.  The fused G side nests every step, since its U blocks
+    // live in registers named by the step; the others run in a loop, so
+    // that a segment may be of any length.
     auto steps = [&](auto self, auto I) __attribute__((always_inline)) {
       constexpr int st = decltype(I)::value;
-      if constexpr (st < FP_STEPS) {
+      if constexpr (st < (PROJ ? FP_STEPS : 2)) {
         if (st < nsteps) {
-          store_q(buf, tc0 + st * FP_T, qv);
-          // The stage's loads (this wave's) must have landed and its V pieces
-          // be written before the barrier.  Vector memory operations complete
-          // in issue order as s_waitcnt counts them, and step 0 issues the
-          // stage's loads before B's loads and the NFLUSH stores of the
-          // previous chunk: at step 1, vmcnt <= NFLUSH covers the stage while
-          // the stores drain.  Other steps wait for everything.
-          if (st == 1)
-            __builtin_amdgcn_s_waitcnt(0x0070 | NFLUSH);  // vmcnt(NFLUSH) lgkmcnt(0)
-          else
-            __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
-          __asm__ volatile("s_barrier" ::: "memory");
-          step(lds + (buf ^ 1) * STAGE, lds + buf * STAGE, st);
-          buf ^= 1;
+          one(st, I);
           self(self, std::integral_constant<int, st + 1>{});
         }
+      } else if constexpr (!PROJ) {
+#pragma unroll 1
+        for (int q = 2; q < nsteps; ++q) one(q, std::integral_constant<int, 2>{});
       }
     };
     steps(steps, std::integral_constant<int, 0>{});
-    hold(acc, m_base, c);
-    if (nsteps == 0) flush();  // no step of the next chunk will
+    if (nsteps == 0) {  // no step of the next chunk will store the zero rows
+      emit(acc, true, m_base, c);
+    }
   }
-  flush();
+  if (nsteps > 0) {
+    emit(acc, c_begin < c_end, (c_end - 1) * FP_MT, c_end - 1);
+  }
 
   // U: lane holds rows 4 (lane >> 4) + i, column lane & 15 of each step's
   // 16 x 16 block: 4 consecutive entries of the column's plane row (tb is a
@@ -891,18 +893,60 @@ __global__ __launch_bounds__(256, 2) void k_factor_project_bf16(const int64_t* _
                                                                 const int32_t* __restrict__ sex,
                                                                 double* __restrict__ part,
                                                                 int64_t part_stride) {
-  factor_pass_bf16<true, 1>(probs, ws, n_prob, sstart, slen, sex, part, part_stride);
+  __shared__ __attribute__((aligned(16))) uint16_t lds[2 * fp_stage(1)];
+  const int p = odp_find_problem(ws, n_prob, blockIdx.x);
+  factor_pass_bf16<true, 1>(probs + (int64_t)p * ODP_FT_FIELDS, blockIdx.x - ws[p], FP_STEPS, lds, sstart, slen, sex,
+                            part, part_stride);
 }
 
-template <int NKB>
-__global__ __launch_bounds__(256, 2) void k_factor_stream_bf16(const int64_t* __restrict__ probs,
-                                                               const int32_t* __restrict__ ws, int n_prob,
+// The streamed factor pass over up to four tables, one per rank block count,
+// in one launch: tables of few workgroups (the shared activations of a short
+// plan) then run beside the others instead of in launches of their own that
+// leave most of the chip idle (two Llama-shaped layers at 4 x 4096 tokens:
+// 957 us in three launches, 772 us in one; four ragged ones at 16 x 1024:
+// 1086 -> 1041 us).  Workgroups take the tables in descending order of rank
+// blocks (the most work per byte first).  A table's workgroups find their row
+// in its map of (row, workgroup within the row) pairs, or by searching
+// work_start: the search is a dozen dependent loads on a table of thousands
+// of rows, during which the workgroup has nothing in flight.
+struct FactorTables {
+  const int64_t* probs[4];  // [k]: the problems of k + 1 rank blocks
+  const int32_t* map[4];    // per workgroup (row, local), or null:
+  const int32_t* ws[4];     // work_start
+  int32_t n_prob[4];
+  int32_t total[4];
+};
+
+__global__ __launch_bounds__(256, 2) void k_factor_stream_bf16(FactorTables T, int max_steps,
                                                                const int32_t* __restrict__ sstart,
                                                                const int32_t* __restrict__ slen,
                                                                const int32_t* __restrict__ sex,
                                                                double* __restrict__ part,
                                                                int64_t part_stride) {
-  factor_pass_bf16<false, NKB>(probs, ws, n_prob, sstart, slen, sex, part, part_stride);
+  __shared__ __attribute__((aligned(16))) uint16_t lds[2 * fp_stage(4)];
+  int bid = blockIdx.x;
+  auto take = [&](auto K) __attribute__((always_inline)) {
+    constexpr int k = decltype(K)::value;
+    if (bid < T.total[k]) {
+      int p, local;
+      if (T.map[k] != nullptr) {
+        p = T.map[k][2 * (int64_t)bid];
+        local = T.map[k][2 * (int64_t)bid + 1];
+      } else {
+        p = odp_find_problem(T.ws[k], T.n_prob[k], bid);
+        local = bid - T.ws[k][p];
+      }
+      factor_pass_bf16<false, k + 1>(T.probs[k] + (int64_t)p * ODP_FT_FIELDS, local, max_steps, lds, sstart, slen,
+                                     sex, part, part_stride);
+      return true;
+    }
+    bid -= T.total[k];
+    return false;
+  };
+  if (take(std::integral_constant<int, 3>{})) return;
+  if (take(std::integral_constant<int, 2>{})) return;
+  if (take(std::integral_constant<int, 1>{})) return;
+  take(std::integral_constant<int, 0>{});
 }
 
 // ---------------------------------------------------------------------------
@@ -1421,14 +1465,50 @@ extern "C" int odp_seg_factor_stream(odp_stream_t stream, const int64_t* problem
     odp_set_error("odp_seg_factor_stream: null segment/partial arrays or part_stride <= 0");
     return ODP_ERR_INVALID_ARGUMENT;
   }
-  hipStream_t s = odp_hip_stream(stream);
-  const dim3 grid(total_blocks), block(256);
-  switch (nkb) {
-    case 1: hipLaunchKernelGGL(k_factor_stream_bf16<1>, grid, block, 0, s, problems, work_start, n_prob, seg_row_start, seg_row_len, seg_example, part, part_stride); break;
-    case 2: hipLaunchKernelGGL(k_factor_stream_bf16<2>, grid, block, 0, s, problems, work_start, n_prob, seg_row_start, seg_row_len, seg_example, part, part_stride); break;
-    default: hipLaunchKernelGGL(k_factor_stream_bf16<3>, grid, block, 0, s, problems, work_start, n_prob, seg_row_start, seg_row_len, seg_example, part, part_stride); break;
-  }
+  FactorTables T = {};
+  T.probs[nkb - 1] = problems;
+  T.ws[nkb - 1] = work_start;
+  T.n_prob[nkb - 1] = n_prob;
+  T.total[nkb - 1] = total_blocks;
+  hipLaunchKernelGGL(k_factor_stream_bf16, dim3(total_blocks), dim3(256), 0, odp_hip_stream(stream), T, FP_STEPS,
+                     seg_row_start, seg_row_len, seg_example, part, part_stride);
   return odp_check_launch("odp_seg_factor_stream");
+}
+
+extern "C" int odp_seg_factor_stream_tables(odp_stream_t stream, const int64_t* const* problems,
+                                            const int32_t* const* block_map, const int32_t* n_prob,
+                                            const int32_t* total_blocks, const int32_t* seg_row_start,
+                                            const int32_t* seg_row_len, const int32_t* seg_example, double* part,
+                                            int64_t part_stride) {
+  const char* what = "odp_seg_factor_stream_tables";
+  if (problems == nullptr || block_map == nullptr || n_prob == nullptr || total_blocks == nullptr) {
+    odp_set_error("%s: null table arrays", what);
+    return ODP_ERR_INVALID_ARGUMENT;
+  }
+  FactorTables T = {};
+  int64_t blocks = 0;
+  for (int k = 0; k < 4; ++k) {
+    int rc = odp_check_table(what, problems[k], block_map[k], n_prob[k], total_blocks[k]);
+    if (rc != ODP_OK) return rc;
+    T.probs[k] = problems[k];
+    T.map[k] = block_map[k];
+    T.n_prob[k] = n_prob[k];
+    T.total[k] = total_blocks[k];
+    blocks += total_blocks[k];
+  }
+  if (blocks == 0) return ODP_OK;
+  if (blocks >= INT32_MAX) {
+    odp_set_error("%s: the tables exceed the int32 workgroup range", what);
+    return ODP_ERR_UNSUPPORTED;
+  }
+  if (seg_row_start == nullptr || seg_row_len == nullptr || seg_example == nullptr || part == nullptr ||
+      part_stride <= 0) {
+    odp_set_error("%s: null segment/partial arrays or part_stride <= 0", what);
+    return ODP_ERR_INVALID_ARGUMENT;
+  }
+  hipLaunchKernelGGL(k_factor_stream_bf16, dim3((unsigned)blocks), dim3(256), 0, odp_hip_stream(stream), T, INT32_MAX,
+                     seg_row_start, seg_row_len, seg_example, part, part_stride);
+  return odp_check_launch(what);
 }
 
 extern "C" int odp_seg_factor(odp_stream_t stream, int dtype, const int64_t* problems,

@@ -5,7 +5,8 @@ for the native kernels and runs the DP step as a fixed sequence of launches
 on the current HIP stream:
 
     odp_project     U_i = G_i B_i^T, V = X [A_1 .. A_k]   (LoRA rank space)
-    odp_seg_factor  per-example dA, dB and their squared-norm partials
+    odp_seg_factor_stream_tables / odp_seg_factor
+                    per-example dA, dB and their squared-norm partials
     odp_sqnorm      squared norms of materialised per-example leaves
     odp_clip_factors  per-example norms -> clip / AUTO-S scales
     odp_scale_sum   clipped sum, cast and normalize_by, into one flat buffer
@@ -18,6 +19,7 @@ buffer and uploaded with one asynchronous copy.
 
 from __future__ import annotations
 
+import ctypes
 import math
 import struct
 import time
@@ -409,6 +411,24 @@ class _Table:
         return probs, ws.astype(np.int32), total
 
 
+class _MappedTable(_Table):
+    """A table of whole rows whose workgroups read their (row, workgroup of
+    the row) from a map instead of searching work_start."""
+
+    def __init__(self, rows: np.ndarray, blocks: np.ndarray, nbytes: int, nflops: int, io: int) -> None:
+        super().__init__(rows.shape[1])
+        self.rows, self.blocks = rows, blocks
+        self.nbytes, self.nflops, self.io_bytes = int(nbytes), int(nflops), int(io)
+
+    def arrays(self) -> tuple[np.ndarray, np.ndarray, int]:
+        total = int(self.blocks.sum())
+        if total >= 2**31 - 1:
+            raise ValueError("launch exceeds the int32 workgroup range; split the batch")
+        row = np.repeat(np.arange(len(self.blocks)), self.blocks)
+        first = np.cumsum(self.blocks) - self.blocks
+        return self.rows, np.stack([row, np.arange(total) - first[row]], axis=1).astype(np.int32), total
+
+
 def _stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 
@@ -506,6 +526,17 @@ def plan_key(*, segments: Segments, leaves: list[LeafOut], clip: ClipSpec, lora_
 # ---------------------------------------------------------------------------
 
 
+# The streamed factor pass: the tables of such a stage (one per rank block
+# count) go out in one launch.
+_STREAM_STAGES = ("factor_stream", "factor_stream_long")
+# Workgroups of the streamed pass a CU holds (two stages of 40 KB each), and
+# how many times over the chip's slots should be filled: below that, segments
+# are split into smaller column groups than odp_seg_factor_stream_groups()'s.
+STREAM_SLOTS_PER_CU = 2
+STREAM_ROUNDS = 4
+# Steps (64 tokens of one 256-column tile) a column group should at least hold.
+STREAM_MIN_STEPS = 8
+
 # Stages launched after the clip factors, in table order.
 _AFTER_CLIP = ("scale_sum", "lin_prescale", "lin_sum", "lin_moments")
 
@@ -518,9 +549,9 @@ class GhostPlan:
 
     ``fuse_g_side``: LoRA sites take the single-pass kernels where they can
     (results are bit-identical either way).  ``stream_factors``: bf16
-    factor problems whose leaves each take a 16-row block of the rank plane
-    (rank <= 16, at most three blocks) take odp_seg_factor_stream instead of
-    odp_seg_factor (bit-identical).  ``linear_pe_bytes``: HBM for
+    factor problems whose leaves each take 16-row blocks of the rank plane of
+    their own take the streamed pass (odp_seg_factor_stream_tables) instead
+    of odp_seg_factor (bit-identical).  ``linear_pe_bytes``: HBM for
     the stored per-example gradients of full-weight sites (bf16); None uses
     half of the free device memory, 0 stores none.  ``prescale_bytes``: at
     most this much of prescaled activations per clipped-sum chunk.
@@ -847,26 +878,24 @@ class GhostPlan:
         # Q planes (U and V) for every chunk, carved from one allocation per dtype.
         q_need: dict[torch.dtype, int] = {}
         chunk_layout = []
-        for ch in chunks:
+        for ci, ch in enumerate(chunks):
             dt = ch[0].x.dtype
-            rtot = sum(s.A.shape[1] for s in ch)
+            cols = self._plane_columns(ch, self._chunk_products[ci])
+            rtot = cols[-1] + ch[-1].A.shape[1]
             rows_alloc = (rtot + 15) // 16 * 16 + 16
             planes = 1  # one plane in the activation dtype (bf16: the reference's rounding of X A, G B^T)
             ldq = (reg.view(ch[0].segments).n_rows + 32 + 7) // 8 * 8
             per = planes * rows_alloc * ldq
             base = q_need.get(dt, 0)
-            chunk_layout.append((dt, rtot, rows_alloc, planes, base, base + per, ldq))
+            chunk_layout.append((dt, cols, rtot, planes, base, base + per, ldq))
             q_need[dt] = base + 2 * per
         self.qbuf = {dt: torch.empty(max(n, 1), dtype=dt, device=dev) for dt, n in q_need.items()}
         # Where each LoRA site's columns of the V and U planes lie (rank_planes).
         self._planes_of: dict[int, tuple] = {}
-        for ci, (ch, (dt, _, _, _, vbase, ubase, ldq)) in enumerate(zip(chunks, chunk_layout)):
-            c0 = 0
+        for ci, (ch, (dt, cols, _, _, vbase, ubase, ldq)) in enumerate(zip(chunks, chunk_layout)):
             for j, s in enumerate(ch):
-                r = s.A.shape[1]
-                self._planes_of[self._chunk_sites[ci][j]] = (dt, vbase, ubase, c0, r, ldq,
+                self._planes_of[self._chunk_sites[ci][j]] = (dt, vbase, ubase, cols[j], s.A.shape[1], ldq,
                                                             reg.view(ch[0].segments).n_rows)
-                c0 += r
 
         # Problem tables, per activation dtype.
         # Tables are keyed by (dtype, rank blocks): one launch per key.
@@ -880,7 +909,7 @@ class GhostPlan:
             return tables.setdefault((dt, (r + 15) // 16), _Table(fields))
 
         elem = {torch.bfloat16: 2, torch.float32: 4}
-        for ci, (ch, (dt, rtot, rows_alloc, planes, vbase, ubase, ldq)) in enumerate(zip(chunks, chunk_layout)):
+        for ci, (ch, (dt, cols, rtot, planes, vbase, ubase, ldq)) in enumerate(zip(chunks, chunk_layout)):
             qb = self.qbuf[dt]
             es = elem[dt]
             v = reg.view(ch[0].segments)
@@ -914,10 +943,9 @@ class GhostPlan:
                     (valid * d_in + rtot * d_in + planes * rtot * valid) * es, 2 * valid * d_in * rtot,
                     io=valid * d_in * es,
                 )
-            c0 = 0
             a_leaves = []
             for j, s in enumerate(ch):
-                r = s.A.shape[1]
+                r, c0 = s.A.shape[1], cols[j]
                 g = ext[("lg", ci, j)]
                 wb = ext[("lwb", ci, j)]
                 d_out = g.shape[1]
@@ -960,7 +988,6 @@ class GhostPlan:
                                            (ln * d_out + 2 * planes * r * ln) * es + r * d_out * es
                                            + (r * d_out * es if j == 0 else 0), ln * d_out * es,
                                            4 * ln * d_out * r))
-                    c0 += r
                     continue
                 if not products:
                     # U_i = G_i B_i^T into columns [c0, c0 + r) of the chunk's U planes.
@@ -981,7 +1008,6 @@ class GhostPlan:
                     tab(ft, dt, r, N.FT_FIELDS).add(frow, n_seg * lib.odp_seg_factor_tiles(dtype_code(dt), d_out, r),
                                                     (valid * d_out + planes * r * valid) * es + n_seg * r * d_out * es,
                                                     2 * valid * d_out * r, io=valid * d_out * es)
-                c0 += r
             if a_leaves:
                 scal = {s.scaling for s in ch if s.a_leaf is not None}
                 if len(scal) != 1:
@@ -997,8 +1023,8 @@ class GhostPlan:
                             arow, n_seg * lib.odp_seg_factor_tiles(dtype_code(dt), d_in, r),
                             (valid * d_in + planes * r * valid) * es + n_seg * r * d_in * es, 2 * valid * d_in * r,
                             io=valid * d_in * es)
-                elif self._streamable(dt, [(c, rk) for _, c, rk in a_leaves], v, x) and (rtot + 15) // 16 <= 3:
-                    # One leaf per 16-row block of U (q/k/v, gate/up at rank 16).
+                elif self._streamable(dt, [(c, rk) for _, c, rk in a_leaves], v, x):
+                    # Every leaf on 16-row blocks of U of its own (q/k/v, gate/up).
                     self._stream_rows(self._a_row(x, d_in, qaddr, ubase, 0, rtot, ldq, sf, n_seg, scal.pop(),
                                                   a_leaves, pe_off, slot_base),
                                       v, d_in, es, planes, stream_rows)
@@ -1016,11 +1042,13 @@ class GhostPlan:
         fp = _Table(N.FT_FIELDS)
         for _, _, row, blocks, nbytes, io, fl in sorted(fused_rows, key=lambda t: (t[0], t[1])):
             fp.add(row, blocks, nbytes, fl, io=io)
-        fst: dict[int, _Table] = {}
-        for nkb in sorted(stream_rows):
-            fst[nkb] = _Table(N.FT_FIELDS)
-            for _, _, row, blocks, nbytes, io, fl in sorted(stream_rows[nkb], key=lambda t: (t[0], t[1])):
-                fst[nkb].add(row, blocks, nbytes, fl, io=io)
+        fst = self._stream_tables(stream_rows)
+        # Plans whose segments all fit odp_factor_project_max_len() rows, and
+        # the others, run the same launch (odp_seg_factor_stream_tables) as
+        # different stages.
+        limit = int(lib.odp_factor_project_max_len())
+        longest = max((int(t[1].max(initial=0)) for rows in stream_rows.values() for t in rows), default=0)
+        stream_stage = "factor_stream" if longest <= limit else "factor_stream_long"
 
         sq = _Table(N.SQ_FIELDS)
         mat_pe: dict[int, torch.Tensor] = {}
@@ -1258,7 +1286,7 @@ class GhostPlan:
             tabs.append(("project", key, pj[key]))
         tabs.append(("factor_project", None, fp))
         for nkb in sorted(fst):
-            tabs.append(("factor_stream", nkb, fst[nkb]))
+            tabs.append((stream_stage, nkb, fst[nkb]))
         for key in sorted(ft, key=lambda k: (str(k[0]), k[1])):
             tabs.append(("factor", key, ft[key]))
         tabs.append(("sqnorm", None, sq))
@@ -1297,11 +1325,21 @@ class GhostPlan:
         self.seg_start, self.seg_len, self.seg_ex = (views[idx[k]] for k in ("seg_start", "seg_len", "seg_ex"))
         self.gstart, self.thr = views[idx["gstart"]], views[idx["thr"]]
         self.guard, self.cls_dt = views[idx["guard"]], views[idx["cls_dt"]]
+        self._stream_arg_cache: dict[str, tuple] = {}
         self.tables = [(name, dt, views[pi], views[wi], n, total) for name, dt, pi, wi, n, total, _ in tab_idx]
         # Per launch, in launch order: (stage, key, workgroups, algorithmic bytes, algorithmic flops,
         # contract bytes: the part of the bytes that reads activations and
         # output gradients or writes the clipped sums).
-        info = [(name, dt, total, nb[0], nb[1], nb[2]) for name, dt, _, _, _, total, nb in tab_idx if total > 0]
+        info: list[tuple] = []
+        for name, dt, _, _, _, total, nb in tab_idx:
+            if total <= 0:
+                continue
+            if info and name in _STREAM_STAGES and info[-1][0] == name:  # one launch takes them all
+                prev = info.pop()
+                keys = (prev[1] if isinstance(prev[1], tuple) else (prev[1],)) + (dt,)
+                info.append((name, keys, prev[2] + total, *(a + b for a, b in zip(prev[3:], nb))))
+            else:
+                info.append((name, dt, total, nb[0], nb[1], nb[2]))
         after_clip = _AFTER_CLIP
         self.launch_info = [i for i in info if i[0] not in after_clip] + [i for i in info if i[0] in after_clip]
 
@@ -1692,34 +1730,69 @@ class GhostPlan:
 
     def _streamable(self, dt: torch.dtype, leaves: list[tuple[int, int]], v: _SegView, p: torch.Tensor) -> bool:
         """Whether a factor problem over P whose leaves sit at these (column
-        in Q, rank) pairs runs as odp_seg_factor_stream: bf16, every leaf on
-        a 16-row block of its own, segments within the kernel's length."""
+        in Q, rank) pairs runs as the streamed pass: bf16, every leaf on
+        16-row blocks of its own, and rows it can address (32-bit offsets
+        within a segment)."""
         if not self.stream_factors or dt != torch.bfloat16:
             return False
-        if not leaves or any(c % 16 or rk > 16 for c, rk in leaves):
-            return False
-        lib = N.load()
-        return v.max_len <= lib.odp_factor_project_max_len() and v.max_len * p.stride(0) * 2 < 2**31
+        return bool(leaves) and all(c % 16 == 0 for c, _ in leaves) and v.max_len * p.stride(0) * 2 < 2**31
+
+    def _plane_columns(self, ch: list[LoraSite], products: bool) -> list[int]:
+        """First column of each site's rank in the chunk's planes.  Planes
+        packed from the seam's products start every site on a 16-column
+        boundary where the chunk still fits one pass, so that the streamed
+        factor pass takes them (bf16); the projection writes its chunk's
+        ranks side by side."""
+        ranks = [s.A.shape[1] for s in ch]
+        if products and self.stream_factors and ch[0].x.dtype == torch.bfloat16:
+            wide = [(r + 15) // 16 * 16 for r in ranks]
+            if sum(wide) <= MAX_RANK_PER_PASS:
+                return [sum(wide[:j]) for j in range(len(ch))]
+        return [sum(ranks[:j]) for j in range(len(ch))]
 
     def _stream_rows(self, row: dict, v: _SegView, M: int, es: int, planes: int, out: dict) -> None:
-        """A factor problem as odp_seg_factor_stream rows: one per segment,
+        """A factor problem as rows of the streamed pass: one per segment,
         each leaf's pe rows at the segment's own offset, so that the launch
         can run the most work per workgroup first."""
-        lib = N.load()
         r = int(row[N.FT_R])
         pe_es = self.pe[torch.bfloat16].element_size()
-        groups = int(lib.odp_seg_factor_stream_groups(M))
         ranks = [(row[N.FT_LEAF0 + 3 * li + 1] >> 16) & 0xFFFF for li in range(int(row[N.FT_NLEAF]))]
-        lst = out.setdefault((r + 15) // 16, [])
-        for j, ln in enumerate(v.segs.lengths):
-            rj = dict(row)
-            rj[N.FT_SEG_FIRST] = v.first + j
-            rj[N.FT_NSEG] = 1
-            for li, rk in enumerate(ranks):
-                rj[N.FT_LEAF0 + 3 * li] = row[N.FT_LEAF0 + 3 * li] + j * rk * M * pe_es
-            rj[N.FT_GROUPS] = groups
-            lst.append((-ln * M / groups, len(lst), rj, groups,
-                        (ln * M + planes * r * ln) * es + sum(ranks) * M * es, ln * M * es, 2 * ln * M * r))
+        base = np.zeros(N.FT_FIELDS, dtype=np.int64)
+        base[list(row)] = list(row.values())
+        j = np.arange(v.n_seg, dtype=np.int64)
+        rows = np.repeat(base[None], v.n_seg, axis=0)
+        rows[:, N.FT_SEG_FIRST] = v.first + j
+        rows[:, N.FT_NSEG] = 1
+        for li, rk in enumerate(ranks):
+            rows[:, N.FT_LEAF0 + 3 * li] += j * (rk * M * pe_es)
+        ln = np.asarray(v.segs.lengths, dtype=np.int64)
+        out.setdefault((r + 15) // 16, []).append(
+            (rows, ln, M, int(((ln * M + planes * r * ln) * es + sum(ranks) * M * es).sum()), int(ln.sum()) * M * es,
+             2 * int(ln.sum()) * M * r))
+
+    def _stream_tables(self, rows: dict[int, list[tuple]]) -> dict[int, _Table]:
+        """The streamed rows as one table per rank block count, most work per
+        workgroup first.  A segment's 256-column tiles go to groups of
+        odp_seg_factor_stream_groups()'s size; while the launch would not
+        fill the chip STREAM_ROUNDS times, to smaller ones of at least
+        STREAM_MIN_STEPS steps."""
+        lib = N.load()
+        slots = STREAM_SLOTS_PER_CU * torch.cuda.get_device_properties(self.device).multi_processor_count \
+            if self.device.type == "cuda" else 1
+        tiles = sum((M + 255) // 256 * int((ln > 0).sum()) for lst in rows.values() for _, ln, M, *_ in lst)
+        per = max(1, tiles // (STREAM_ROUNDS * slots))
+        out: dict[int, _Table] = {}
+        for nkb in sorted(rows):
+            work = []
+            for arr, ln, M, *_ in rows[nkb]:
+                n = (M + 255) // 256
+                size = np.maximum(per, -(-STREAM_MIN_STEPS // np.maximum((ln + 63) // 64, 1)))
+                arr[:, N.FT_GROUPS] = np.maximum(int(lib.odp_seg_factor_stream_groups(M)), -(-n // size))
+                work.append(ln * M / arr[:, N.FT_GROUPS])
+            order = np.argsort(-np.concatenate(work), kind="stable")
+            arr = np.concatenate([t[0] for t in rows[nkb]])[order]
+            out[nkb] = _MappedTable(arr, arr[:, N.FT_GROUPS], *(sum(t[k] for t in rows[nkb]) for k in (3, 5, 4)))
+        return out
 
     def _a_row(self, x, d_in, qaddr, ubase, col0, r, ldq, seg_first, n_seg, scaling, leaves, pe_off, slot_base):
         row = {
@@ -1769,6 +1842,19 @@ class GhostPlan:
         """The per-example factor gradients each LoRA leaf stored ([n_seg * r * M], parameter dtype)."""
         return [self.pe[dt][o : o + n] for dt, o, n in self._pe_slices]
 
+    def _stream_args(self, stage: str) -> tuple:
+        """Host arrays of the stage's tables for odp_seg_factor_stream_tables."""
+        args = self._stream_arg_cache.get(stage)
+        if args is None:
+            by_nkb = {t[1]: t for t in self.tables if t[0] == stage and t[5] > 0}
+            rows = [by_nkb.get(k + 1) for k in range(4)]
+            args = self._stream_arg_cache[stage] = (
+                (ctypes.c_void_p * 4)(*[t[2].data_ptr() if t else None for t in rows]),
+                (ctypes.c_void_p * 4)(*[t[3].data_ptr() if t else None for t in rows]),
+                (ctypes.c_int32 * 4)(*[t[4] if t else 0 for t in rows]),
+                (ctypes.c_int32 * 4)(*[t[5] if t else 0 for t in rows]))
+        return args
+
     # -- execution -------------------------------------------------------------
     def run(self, events: dict | None = None, launch_log: list | None = None) -> GhostResult:
         """Launch the step on the current stream.
@@ -1813,11 +1899,10 @@ class GhostPlan:
                                                    self.seg_start.data_ptr(), self.seg_len.data_ptr(),
                                                    self.seg_ex.data_ptr(), self.part.data_ptr(),
                                                    self.n_slots), name)
-            elif name == "factor_stream":
-                N.check(lib.odp_seg_factor_stream(s, probs.data_ptr(), ws.data_ptr(), n, total,
-                                                  self.seg_start.data_ptr(), self.seg_len.data_ptr(),
-                                                  self.seg_ex.data_ptr(), self.part.data_ptr(),
-                                                  self.n_slots, dt), name)
+            elif name in _STREAM_STAGES:
+                N.check(lib.odp_seg_factor_stream_tables(s, *self._stream_args(name), self.seg_start.data_ptr(),
+                                                         self.seg_len.data_ptr(), self.seg_ex.data_ptr(),
+                                                         self.part.data_ptr(), self.n_slots), name)
             elif name == "factor":
                 N.check(lib.odp_seg_factor(s, dtype_code(dt[0]), probs.data_ptr(), ws.data_ptr(), n, total,
                                            self.seg_start.data_ptr(), self.seg_len.data_ptr(),
@@ -1840,13 +1925,15 @@ class GhostPlan:
         # on MI355X.)
         names = [t[0] for t in live]
         for idx, (name, dt, probs, ws, n, total) in enumerate(live):
+            if name in _STREAM_STAGES and name in names[:idx]:
+                continue  # went out with the stage's first table
             if name in ev and name not in names[:idx]:
                 ev[name][0].record(main)
             end_ev = mark(name, dt, main)
             launch(name, dt, probs, ws, n, total, stream)
             if end_ev is not None:
                 end_ev.record(main)
-            if name in ev and name not in names[idx + 1:]:
+            if name in ev and (name in _STREAM_STAGES or name not in names[idx + 1:]):
                 ev[name][1].record(main)
         if "clip" in ev:
             ev["clip"][0].record()

@@ -1,0 +1,122 @@
+"""The streamed factor pass beyond one 16-row block and one fixed length.
+
+odp_seg_factor_stream_tables takes segments of any length, leaves that span
+several 16-row blocks of the rank plane (rank up to 64), chunks of several
+sites whose ranks are packed on 16-column boundaries, and tables of several
+rank block counts in one launch.  Its rows, partial slots and therefore every
+output of a plan equal the tiled pass's (stream_factors=False) bit for bit:
+both form the same 32-token MFMA blocks in the same order.  The tiled pass
+is checked against the oracle elsewhere (test_gpu_kernels.py,
+test_gpu_configs.py).
+"""
+
+from __future__ import annotations
+
+import ctypes
+import math
+
+import pytest
+import torch
+
+from opaque_amd import _native as N
+from opaque_amd.engine import ClipSpec, GhostPlan, LeafOut, LoraSite, Segments
+from opaque_amd.guard import guard_constants, leaf_guards
+
+DEV = "cuda"
+
+# d_in, [(d_out, rank)] per activation; lengths of the examples
+LIMIT = 1081  # odp_factor_project_max_len()
+CASES = {
+    # one step past the fixed-length kernels' bound, steps not a multiple of 64, an empty and a one-row segment
+    "long": ([(264, [(520, 16)])], [LIMIT + 1, 0, 1, 2 * LIMIT + 9]),
+    "rank20": ([(136, [(72, 20)])], [96, 33, 1, 70]),
+    "rank32": ([(520, [(264, 32)])], [65, 0, 64, 63]),
+    "rank64": ([(264, [(4360, 64)])], [129, 88, 5, 0]),  # 18 tiles in several groups, the last partial
+    "rank64_long": ([(72, [(136, 64)])], [LIMIT + 70, 3, 700, 0]),
+    "shared_r8": ([(256, [(256, 8), (64, 8), (64, 8)])], [128, 77, 0, 9]),  # three blocks of 8 of 16 rows
+    "shared_r24": ([(128, [(264, 24), (72, 24)])], [96, 50, 3, 64]),  # two leaves of two blocks each
+    "shared_four": ([(128, [(64, 4), (72, 16), (80, 12), (88, 1)])], [70, 64, 1, 0]),
+    "shared_r20_tiled": ([(128, [(64, 20), (72, 20), (80, 20)])], [70, 64, 1, 0]),  # 96 columns: packed side by side
+    "mixed": ([(256, [(256, 16), (64, 16), (64, 16)]), (72, [(200, 64)]), (512, [(128, 16)]),
+               (136, [(264, 32)])], [200, 64, 31, 129]),  # tables of 1, 2, 3 and 4 blocks
+}
+
+
+def _case(name, scalings=(2.0,)):
+    acts, lengths = CASES[name]
+    g = torch.Generator(device=DEV).manual_seed(sum(map(ord, name)))
+    T = max(lengths)
+    n_rows = len(lengths) * T
+    seg = Segments.padded(len(lengths), T, lengths)
+
+    def rnd(*shape, scale=1.0):
+        return (torch.randn(*shape, device=DEV, generator=g) * scale).to(torch.bfloat16)
+
+    sites, leaves = [], []
+    for d_in, outs in acts:
+        x = rnd(n_rows, d_in)
+        for k, (d_out, r) in enumerate(outs):
+            gt, A, B = rnd(n_rows, d_out, scale=0.3), rnd(d_in, r, scale=1 / math.sqrt(d_in)), rnd(r, d_out, scale=0.05)
+            n = len(leaves)
+            leaves += [LeafOut((d_in, r), torch.bfloat16), LeafOut((r, d_out), torch.bfloat16)]
+            sites.append(LoraSite(x, gt, A, B, scalings[k % len(scalings)], a_leaf=n, b_leaf=n + 1, v=x @ A,
+                                  u=gt @ B.t().contiguous()))
+    return seg, sites, leaves
+
+
+def _plan(seg, sites, leaves, stream):
+    _, rnd = leaf_guards([lf.shape for lf in leaves], [torch.bfloat16] * len(leaves))
+    rel, ab = guard_constants(torch.bfloat16, rnd)
+    clip = ClipSpec(mode=N.CLIP_AUTOS, thresholds=[1.0], effective=1.0, gamma=0.01, normalize_by=2.0,
+                    guards=[(rel, ab, torch.bfloat16)])
+    return GhostPlan(segments=seg, leaves=leaves, clip=clip, lora_sites=sites, device=DEV, stream_factors=stream)
+
+
+def _outputs(plan):
+    res = plan.run()
+    torch.cuda.synchronize()
+    return [t.clone() for t in plan.pe_views()] + [t.clone() for t in res.leaves] + [res.norms.clone(),
+                                                                                   plan.part.sum(1)]
+
+
+def _check(name, scalings=(2.0,)):
+    assert int(N.load().odp_factor_project_max_len()) == LIMIT
+    seg, sites, leaves = _case(name, scalings)
+    off, on = _plan(seg, sites, leaves, False), _plan(seg, sites, leaves, True)
+    stages = {t[0] for t in on.tables if t[5] > 0}
+    assert stages & {"factor_stream", "factor_stream_long"} and ("factor" in stages) == name.endswith("tiled"), stages
+    for k, (a, b) in enumerate(zip(_outputs(on), _outputs(off))):
+        assert torch.isfinite(a.float()).all(), k
+        # The partial slots are summed here in another order than the slots'.
+        assert torch.equal(a, b) if a.dtype != torch.float64 else torch.allclose(a, b, rtol=1e-13), k
+    return on
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_streamed_tables_equal_the_tiled_pass(name):
+    print(f"streamed factor tables: {name}", flush=True)
+    on = _check(name)
+    if name == "mixed":
+        assert {t[1] for t in on.tables if t[0] == "factor_stream" and t[5] > 0} == {1, 2, 3, 4}
+        assert [i[1] for i in on.launch_info if i[0] == "factor_stream"] == [(1, 2, 3, 4)]
+
+
+@pytest.mark.gpu
+def test_sites_of_different_scalings_stream_their_own_rows():
+    print("streamed factor tables: two scalings", flush=True)
+    _check("shared_r24", (2.0, 0.5))
+
+
+def test_argument_checks():
+    lib = N.load()
+    null, bad = (ctypes.c_void_p * 4)(), (ctypes.c_void_p * 4)(8, None, None, None)
+    zero, one = (ctypes.c_int32 * 4)(), (ctypes.c_int32 * 4)(1, 0, 0, 0)
+    call = lib.odp_seg_factor_stream_tables
+    assert call(None, null, null, zero, zero, None, None, None, None, 1) == N.ODP_OK  # no work
+    assert call(None, None, null, zero, zero, None, None, None, None, 1) == N.ERR_INVALID_ARGUMENT
+    assert call(None, null, null, one, one, None, None, None, None, 1) == N.ERR_INVALID_ARGUMENT
+    assert call(None, bad, bad, one, one, None, None, None, None, 1) == N.ERR_INVALID_ARGUMENT
+    assert "null segment" in lib.odp_last_error().decode()
+    assert call(None, bad, bad, zero, one, 8, 8, 8, 8, 1) == N.ERR_INVALID_ARGUMENT  # work without problems
+    assert call(None, bad, bad, one, one, 8, 8, 8, 8, 0) == N.ERR_INVALID_ARGUMENT  # part_stride
