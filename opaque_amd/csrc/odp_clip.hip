@@ -19,22 +19,8 @@ constexpr int CL_DEPTH = 8;      // loads in flight per thread (a power of two)
 constexpr int CL_MAX_GROUPS = 1024;
 static_assert(CL_MAX_GROUPS <= CL_THREADS, "thread g finishes group g");
 constexpr int SS_THREADS = 256;
-constexpr int SS_ELEMS = 8;  // elements per thread
-
-// Workgroup sum in a fixed order (a fixed tree within each wave by DPP and
-// lane reads, then the wave sums in wave order), so that runs are bitwise
-// reproducible.  The result is valid in every thread.
-__device__ __forceinline__ double block_sum_fixed(double v, double* red) {
-  v = rows_sum4(row_sum16(v));
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) red[wave] = v;
-  __syncthreads();
-  double t = 0.0;
-#pragma unroll
-  for (int w = 0; w < CL_THREADS / 64; ++w) t += red[w];
-  __syncthreads();
-  return t;
-}
+constexpr int SS_ELEMS = 4;  // elements per thread of the element-wise form
+#define ODP_CONST __attribute__((address_space(4)))  // uniform values through the scalar path
 
 // The scale as the leaf dtype holds it (float64 leaves keep every bit).
 __device__ __forceinline__ double finalize_scale(double ratio, double rel, double abs_, int clamp_one,
@@ -51,7 +37,12 @@ __device__ __forceinline__ double finalize_scale(double ratio, double rel, doubl
 // The sum of an example's partials (a few hundred KB on Llama-shaped
 // models) is bound by what one CU can have in flight, so each thread issues
 // CL_DEPTH 16-byte loads at once; the order of additions is fixed (it does
-// not depend on which loads are masked), so runs are bitwise reproducible.
+// not depend on which loads are masked: a fixed tree within each wave by DPP
+// and lane reads, then the group's waves in order), so runs are bitwise
+// reproducible.  Several groups are summed side by side, the 16 waves split
+// evenly among them: one after the other, each by the whole workgroup, they
+// are a chain of load latencies and barriers (14 groups of 584 partials: 19
+// us, 7 us side by side; one group: 6 us either way).
 // `status` (optional): a word that k_sqnorm sets when it dropped a write
 // outside the partials; every example then gets a NaN norm, zero scales and
 // clear masks, since the partials are incomplete.
@@ -88,42 +79,57 @@ __global__ __launch_bounds__(CL_THREADS) void k_clip_factors(
   if (t < 2 * n_cls) sguard[t] = guard[t];
   if (t < n_cls) scls[t] = cls_dtype[t];
 
-  for (int g = 0; g < n_groups; ++g) {
-    const int64_t hi = gstart[g + 1];
+  // Waves per group: 16 for one group, halved until the groups fit side by
+  // side (one wave each beyond 8 groups, in rounds of 16 groups).
+  constexpr int NWAVE = CL_THREADS / 64;
+  int wpg = NWAVE;
+  while (wpg > 1 && wpg * n_groups > NWAVE) wpg >>= 1;
+  const int wave = t >> 6, nth = 64 * wpg, tg = t & (nth - 1);
+  for (int g0 = 0; g0 < n_groups; g0 += NWAVE / wpg) {
+    const int g = g0 + wave / wpg;
     double a[CL_DEPTH];
 #pragma unroll
     for (int q = 0; q < CL_DEPTH; ++q) a[q] = 0.0;
-    // Slots are read in 16-byte pairs from the first 16-byte aligned one
-    // (by address, so any 8-byte aligned partials buffer works; a leading
-    // and a trailing odd slot go to thread 0), and every load of a round is
-    // issued before the first add (masked past the group's end).
-    const int64_t lo = gstart[g];
-    int64_t la = lo + (int64_t)((((uintptr_t)(row + lo)) >> 3) & 1u);
-    la = la < hi ? la : hi;
-    const int64_t npair = (hi - la) >> 1;
-    if (t == 0) {
-      if (lo < la) a[0] += row[lo];
-      if (la + 2 * npair < hi) a[1] += row[hi - 1];
+    if (g < n_groups) {
+      // Slots are read in 16-byte pairs from the first 16-byte aligned one
+      // (by address, so any 8-byte aligned partials buffer works; a leading
+      // and a trailing odd slot go to the group's first thread), and every
+      // load of a round is issued before the first add (masked past the
+      // group's end).
+      const int64_t lo = gstart[g], hi = gstart[g + 1];
+      int64_t la = lo + (int64_t)((((uintptr_t)(row + lo)) >> 3) & 1u);
+      la = la < hi ? la : hi;
+      const int64_t npair = (hi - la) >> 1;
+      if (tg == 0) {
+        if (lo < la) a[0] += row[lo];
+        if (la + 2 * npair < hi) a[1] += row[hi - 1];
+      }
+      const double2* pr = (const double2*)(row + la);
+      for (int64_t q0 = tg; q0 < npair; q0 += CL_DEPTH * nth) {
+        double2 v[CL_DEPTH];
+#pragma unroll
+        for (int q = 0; q < CL_DEPTH; ++q)
+          v[q] = q0 + q * nth < npair ? pr[q0 + q * nth] : double2{0.0, 0.0};
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < CL_DEPTH; ++q) a[q] = (a[q] + v[q].x) + v[q].y;
+      }
+      // Pairwise over the accumulators, in a fixed order.
+#pragma unroll
+      for (int w = CL_DEPTH / 2; w > 0; w >>= 1)
+#pragma unroll
+        for (int q = 0; q < w; ++q) a[q] = a[2 * q] + a[2 * q + 1];
     }
-    const double2* pr = (const double2*)(row + la);
-    for (int64_t q0 = t; q0 < npair; q0 += CL_DEPTH * CL_THREADS) {
-      double2 v[CL_DEPTH];
-#pragma unroll
-      for (int q = 0; q < CL_DEPTH; ++q)
-        v[q] = q0 + q * CL_THREADS < npair ? pr[q0 + q * CL_THREADS] : double2{0.0, 0.0};
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int q = 0; q < CL_DEPTH; ++q) a[q] = (a[q] + v[q].x) + v[q].y;
+    const double ws = rows_sum4(row_sum16(a[0]));
+    if ((t & 63) == 0) red[wave] = ws;
+    __syncthreads();
+    if (g < n_groups && tg == 0) {
+      double tot = 0.0;
+      for (int w = 0; w < wpg; ++w) tot += red[wave + w];
+      gsq[g] = tot;
     }
-    // Pairwise over the accumulators, in a fixed order.
-#pragma unroll
-    for (int w = CL_DEPTH / 2; w > 0; w >>= 1)
-#pragma unroll
-      for (int q = 0; q < w; ++q) a[q] = a[2 * q] + a[2 * q + 1];
-    const double tot = block_sum_fixed(a[0], red);
-    if (t == 0) gsq[g] = tot;
+    __syncthreads();
   }
-  __syncthreads();
 
   if (t == 0) {
     double total = 0.0;
@@ -151,8 +157,8 @@ __global__ __launch_bounds__(CL_THREADS) void k_clip_factors(
 // in segment order.  Each term is scale * value rounded to the value's dtype
 // (clip_pytree's `scale.to(dtype) * leaf`), accumulated in float32, or in
 // float64 (Acc = double) for float64 values or a float64 compute dtype.
-// This element-wise form serves float16/float64, the float64 sums and raw
-// sums; the kernel below vectorises float32/bfloat16.  `raw`: the values
+// This element-wise form serves float64, the float64 sums and raw sums; the
+// form below vectorises float32, bfloat16 and float16.  `raw`: the values
 // are already scaled (a caller's scale function): each is summed as it is,
 // with scale 1 and no nan_to_num, as the reference sums a scale function's
 // output (_clipped_fun.py:673-700, 777-782).
@@ -208,20 +214,21 @@ __device__ __forceinline__ void scale_sum_generic(const void* pe, int pdt, int64
   }
 }
 
-// One clipped-sum term per element: the per-example value with non-finite
-// entries zeroed (nan_to_num), times the scale, rounded to bf16 when the
-// values are bf16 (scale.to(dtype) * leaf); accumulated in float32.
-template <bool SECOND, bool BF>
+// One clipped-sum term: the per-example value with non-finite entries zeroed
+// (nan_to_num), times the scale, rounded to the values' dtype when it is a
+// 16-bit one (scale.to(dtype) * leaf); accumulated in float32.
+template <int PDT>
+__device__ __forceinline__ float ss_round(float v) {
+  if (PDT == ODP_DTYPE_BF16) return odp_round_bf16(v);
+  if (PDT == ODP_DTYPE_F16) return (float)(_Float16)v;
+  return v;
+}
+template <bool SECOND, int PDT>
 __device__ __forceinline__ void ss_term(float v, float c, float& acc, float& acc2) {
   if (!isfinite(v)) v = 0.f;
-  float y = __fmul_rn(c, v);
-  if (BF) y = odp_round_bf16(y);
+  const float y = ss_round<PDT>(__fmul_rn(c, v));
   acc = __fadd_rn(acc, y);
-  if (SECOND) {
-    float yy = __fmul_rn(y, y);
-    if (BF) yy = odp_round_bf16(yy);
-    acc2 = __fadd_rn(acc2, yy);
-  }
+  if (SECOND) acc2 = __fadd_rn(acc2, ss_round<PDT>(__fmul_rn(y, y)));
 }
 
 // The sum cast to the output dtype, then divided in it (the reference's order).
@@ -231,158 +238,199 @@ __device__ __forceinline__ float ss_finish(float acc, float normalize_by, int od
   return x;
 }
 
-// 8 consecutive outputs: one 16-byte store (bf16) or two (f32).
-__device__ __forceinline__ void ss_put8(void* dst, int64_t o, int odt, const float (&y)[SS_ELEMS]) {
-  if (odt == ODP_DTYPE_BF16) {
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    u32x4 w;
-    w.x = (uint32_t)odp_f2bf(y[0]) | ((uint32_t)odp_f2bf(y[1]) << 16);
-    w.y = (uint32_t)odp_f2bf(y[2]) | ((uint32_t)odp_f2bf(y[3]) << 16);
-    w.z = (uint32_t)odp_f2bf(y[4]) | ((uint32_t)odp_f2bf(y[5]) << 16);
-    w.w = (uint32_t)odp_f2bf(y[6]) | ((uint32_t)odp_f2bf(y[7]) << 16);
-    odp_gstore((u32x4*)((uint16_t*)dst + o), w);
-  } else {
-    odp_gstore((f32x4_t*)((float*)dst + o), f32x4_t{y[0], y[1], y[2], y[3]});
-    odp_gstore((f32x4_t*)((float*)dst + o + 4), f32x4_t{y[4], y[5], y[6], y[7]});
-  }
-}
-
-// The sums take segments SS_SG at a time: the scales and values of a group
-// are all loaded before the first of them is accumulated, so several loads
-// are in flight per thread, and the accumulation order (and so every sum)
-// is that of one segment at a time.  Stored per-example values are read
-// once, non-temporally.
-constexpr int SS_SG = 4;
 typedef uint32_t ss_u32x4 __attribute__((ext_vector_type(4)));
 
-// Eight consecutive values at element `at` (bf16: one 16-byte load).
-template <bool BF>
-__device__ __forceinline__ void ss_load8_row(const void* pe, int64_t at, float (&v)[SS_ELEMS]) {
-  if (BF) {
-    const ss_u32x4 w = __builtin_nontemporal_load((const ss_u32x4*)((const uint16_t*)pe + at));
+// Values per 16-byte piece.
+template <int PDT>
+__host__ __device__ constexpr int ss_vec() { return PDT == ODP_DTYPE_F32 ? 4 : 8; }
+
+template <int PDT>
+__device__ __forceinline__ void ss_unpack(const ss_u32x4& w, float (&v)[ss_vec<PDT>()]) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < 4; ++i) {
+    if (PDT == ODP_DTYPE_F32) {
+      v[i] = __uint_as_float(w[i]);
+    } else if (PDT == ODP_DTYPE_BF16) {
       v[2 * i] = __uint_as_float(w[i] << 16);
       v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    } else {
+      v[2 * i] = (float)__builtin_bit_cast(_Float16, (uint16_t)w[i]);
+      v[2 * i + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w[i] >> 16));
     }
+  }
+}
+
+// V consecutive outputs (finished values): 16-byte stores where `vec`.
+template <int V>
+__device__ __forceinline__ void ss_put(void* dst, int64_t o, int odt, bool vec, const float (&y)[V]) {
+  if (!vec) {
+#pragma unroll
+    for (int i = 0; i < V; ++i) odp_store_from_float(dst, o + i, odt, y[i]);
+  } else if (odt == ODP_DTYPE_F32) {
+#pragma unroll
+    for (int i = 0; i < V; i += 4)
+      odp_gstore((f32x4_t*)((float*)dst + o + i), f32x4_t{y[i], y[i + 1], y[i + 2], y[i + 3]});
   } else {
-    const f32x4_t a = __builtin_nontemporal_load((const f32x4_t*)((const float*)pe + at));
-    const f32x4_t b = __builtin_nontemporal_load((const f32x4_t*)((const float*)pe + at + 4));
+    uint32_t w[V / 2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[i] = a[i];
-      v[4 + i] = b[i];
+    for (int i = 0; i < V / 2; ++i) {
+      if (odt == ODP_DTYPE_BF16)
+        w[i] = (uint32_t)odp_f2bf(y[2 * i]) | ((uint32_t)odp_f2bf(y[2 * i + 1]) << 16);
+      else
+        w[i] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)y[2 * i]) |
+               ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)y[2 * i + 1]) << 16);
+    }
+    if (V == 8)
+      odp_gstore((ss_u32x4*)((uint16_t*)dst + o), ss_u32x4{w[0], w[1], w[V / 2 - 2], w[V / 2 - 1]});
+    else {
+      typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+      odp_gstore((u32x2*)((uint16_t*)dst + o), u32x2{w[0], w[1]});
     }
   }
 }
 
-// Eight values M elements apart from element `base` (ranks k0.. of a column).
-template <bool BF>
-__device__ __forceinline__ void ss_load8_col(const void* pe, int64_t base, int64_t M, float (&v)[SS_ELEMS]) {
-#pragma unroll
-  for (int i = 0; i < SS_ELEMS; ++i)
-    v[i] = BF ? odp_bf2f(__builtin_nontemporal_load((const uint16_t*)pe + base + i * M))
-              : __builtin_nontemporal_load((const float*)pe + base + i * M);
-}
+// The sums of float32, bfloat16 and float16 values into float32, bfloat16
+// or float16 outputs, a few segments at a time: the values of a group are
+// all loaded before the first of them is accumulated, and the accumulation
+// order (and so every sum) is that of one segment at a time.  The clip
+// factors come by scalar loads issued behind the values'.  Stored
+// per-example values are read once, non-temporally.  A workgroup takes
+// tiles b, b + nblk, ... of the leaf, each SS_THREADS pieces of V values:
+//   rows: consecutive elements, one 16-byte load per piece and segment
+//         (VEC false, a row length or an address off the 16-byte grid: one
+//         element per thread, so pieces of one value);
+//   transposed ([rank][M] values, [M][rank] outputs): `rank` rows of a run
+//         of columns, turned around through LDS so that the outputs leave as
+//         one contiguous run.
+template <int PDT>
+__host__ __device__ constexpr int ss_sg() { return PDT == ODP_DTYPE_F32 ? 8 : 4; }  // 8 KB a wave and group
+// A transposed tile's element in LDS: one word of skew every 32, so that the
+// column writes (strides of V * rank words) spread over the banks and aligned
+// runs of 8 stay contiguous.
+__device__ __forceinline__ int ss_at(int i) { return i + (i >> 5); }
 
-// bf16/f32 values and outputs, E a multiple of 8: a thread sums the 8
-// consecutive elements e0.. over the segments (16-byte loads for bf16).
-template <bool SECOND, bool BF>
-__device__ __forceinline__ void scale_sum_rows(const void* pe, int64_t E, int64_t M, int rank, int64_t e0, int n_seg,
-                                               int seg_first, const int32_t* __restrict__ sex,
+template <bool SECOND, int PDT, bool VEC>
+__device__ __forceinline__ void scale_sum_fast(const void* pe, int64_t M, int rank, bool transpose, int b, int nblk,
+                                               int n_seg, int seg_first, const int32_t* __restrict__ sex,
                                                const double* __restrict__ sc, float normalize_by, void* out,
-                                               void* out2, int odt, int transpose) {
-  float acc[SS_ELEMS], acc2[SS_ELEMS];
-#pragma unroll
-  for (int i = 0; i < SS_ELEMS; ++i) acc[i] = acc2[i] = 0.f;
-  int s = 0;
-  for (; s + SS_SG <= n_seg; s += SS_SG) {
-    float c[SS_SG], v[SS_SG][SS_ELEMS];
-#pragma unroll
-    for (int q = 0; q < SS_SG; ++q) {
-      c[q] = (float)sc[sex[seg_first + s + q]];
-      ss_load8_row<BF>(pe, (int64_t)(s + q) * E + e0, v[q]);
+                                               void* out2, int odt, float* tile) {
+  constexpr int V = VEC ? ss_vec<PDT>() : 1, ES = PDT == ODP_DTYPE_F32 ? 4 : 2;
+  const int tid = threadIdx.x;
+  const int64_t E = M * rank;
+  // Transposed: columns per tile (a multiple of V), pieces per row.
+  const int cols = transpose ? SS_THREADS * V / rank / V * V : 0, ppr = transpose ? cols / V : 1;
+  const int64_t ntile = transpose ? (M + cols - 1) / cols : (E + SS_THREADS * V - 1) / (SS_THREADS * V);
+  const ODP_CONST int32_t* ex = (const ODP_CONST int32_t*)(sex + seg_first);
+  const ODP_CONST double* csc = (const ODP_CONST double*)sc;
+  for (int64_t t = b; t < ntile; t += nblk) {
+    // Element of segment 0 this thread starts at, and how many it has.
+    int64_t e0;
+    bool on;
+    const int k = transpose ? tid / ppr : 0;
+    if (transpose) {
+      const int64_t m = t * cols + (int64_t)(tid % ppr) * V;
+      e0 = (int64_t)k * M + m;
+      on = k < rank && m < M;
+    } else {
+      e0 = t * (SS_THREADS * V) + tid * V;
+      on = e0 < E;
     }
+    float acc[V], acc2[V];
 #pragma unroll
-    for (int q = 0; q < SS_SG; ++q)
+    for (int i = 0; i < V; ++i) acc[i] = acc2[i] = 0.f;
+    // Segments [s, s + n), n <= SG, all loaded before the first is added.
+    // The barriers keep the compiler from widening every piece at once.
+    constexpr int SG = VEC ? ss_sg<PDT>() : 8;
+    auto group = [&](int s, int n) __attribute__((always_inline)) {
+      float c[SG], v[VEC ? V : SG];
+      ss_u32x4 w[VEC ? SG : 1];
+      const char* src = (const char*)pe + ((int64_t)s * E + e0) * ES;
 #pragma unroll
-      for (int i = 0; i < SS_ELEMS; ++i) ss_term<SECOND, BF>(v[q][i], c[q], acc[i], acc2[i]);
-  }
-  for (; s < n_seg; ++s) {
-    const float c = (float)sc[sex[seg_first + s]];
-    float v[SS_ELEMS];
-    ss_load8_row<BF>(pe, (int64_t)s * E + e0, v);
+      for (int q = 0; q < SG; ++q, src += E * ES)
+        if (q < n) {
+          if constexpr (VEC)
+            w[q] = __builtin_nontemporal_load((const ODP_GMEM ss_u32x4*)(const ODP_GMEM void*)src);
+          else
+            v[q] = odp_load_as_float(src, 0, PDT);
+        }
 #pragma unroll
-    for (int i = 0; i < SS_ELEMS; ++i) ss_term<SECOND, BF>(v[i], c, acc[i], acc2[i]);
-  }
-  float x[SS_ELEMS], x2[SS_ELEMS];
+      for (int q = 0; q < SG; ++q)
+        if (q < n) c[q] = (float)csc[ex[s + q]];
 #pragma unroll
-  for (int i = 0; i < SS_ELEMS; ++i) {
-    x[i] = ss_finish(acc[i], normalize_by, odt);
-    if (SECOND) x2[i] = ss_finish(acc2[i], normalize_by, odt);
-  }
-  if (!transpose) {
-    ss_put8(out, e0, odt, x);
-    if (SECOND) ss_put8(out2, e0, odt, x2);
-    return;
-  }
+      for (int q = 0; q < SG; ++q) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (q < n) {
+          if constexpr (VEC) {
+            ss_unpack<PDT>(w[q], v);
 #pragma unroll
-  for (int i = 0; i < SS_ELEMS; ++i) {
-    const int64_t e = e0 + i;
-    const int64_t k = e / M, m = e - k * M;
-    odp_store_from_float(out, m * rank + k, odt, x[i]);
-    if (SECOND) odp_store_from_float(out2, m * rank + k, odt, x2[i]);
-  }
-}
-
-// Transposed outputs: a thread sums ranks k0..k0+7 of column m (e_first is
-// element (k0, m), rows M apart) and stores them at o = m * rank + k0.
-template <bool SECOND, bool BF>
-__device__ __forceinline__ void scale_sum_cols(const void* pe, int64_t E, int64_t M, int64_t e_first, int n_seg,
-                                               int seg_first, const int32_t* __restrict__ sex,
-                                               const double* __restrict__ sc, float normalize_by, void* out,
-                                               void* out2, int odt, int64_t o) {
-  float acc[SS_ELEMS], acc2[SS_ELEMS];
-#pragma unroll
-  for (int i = 0; i < SS_ELEMS; ++i) acc[i] = acc2[i] = 0.f;
-  int s = 0;
-  for (; s + SS_SG <= n_seg; s += SS_SG) {
-    float c[SS_SG], v[SS_SG][SS_ELEMS];
-#pragma unroll
-    for (int q = 0; q < SS_SG; ++q) {
-      c[q] = (float)sc[sex[seg_first + s + q]];
-      ss_load8_col<BF>(pe, (int64_t)(s + q) * E + e_first, M, v[q]);
+            for (int i = 0; i < V; ++i) ss_term<SECOND, PDT>(v[i], c[q], acc[i], acc2[i]);
+          } else {
+            ss_term<SECOND, PDT>(v[q], c[q], acc[0], acc2[0]);
+          }
+        }
+      }
+    };
+    if (on) {
+      int s = 0;
+      for (; s + SG <= n_seg; s += SG) group(s, SG);
+      if (s < n_seg) group(s, n_seg - s);
     }
+    float x[V], x2[V];
 #pragma unroll
-    for (int q = 0; q < SS_SG; ++q)
+    for (int i = 0; i < V; ++i) {
+      x[i] = ss_finish(acc[i], normalize_by, odt);
+      if (SECOND) x2[i] = ss_finish(acc2[i], normalize_by, odt);
+    }
+    if constexpr (!VEC) {
+      if (!on) continue;
+      odp_store_from_float(out, e0, odt, x[0]);
+      if (SECOND) odp_store_from_float(out2, e0, odt, x2[0]);
+    } else if (!transpose) {
+      const int oes = odp_dtype_size(odt);
+      if (on) {
+        ss_put<V>(out, e0, odt, (((uintptr_t)out + e0 * oes) & (V * oes - 1) & 15) == 0, x);
+        if (SECOND) ss_put<V>(out2, e0, odt, (((uintptr_t)out2 + e0 * oes) & (V * oes - 1) & 15) == 0, x2);
+      }
+    } else {
+      // Tile as [column][rank]: the run out[t * cols * rank ...).
+      const int64_t m0 = t * cols;
+      const int run = (int)((M - m0 < cols ? M - m0 : cols) * rank);
+#pragma unroll 1
+      for (int h = 0; h < (SECOND ? 2 : 1); ++h) {
+        __syncthreads();
+        if (on) {
+          const int c0 = (tid % ppr) * V;
 #pragma unroll
-      for (int i = 0; i < SS_ELEMS; ++i) ss_term<SECOND, BF>(v[q][i], c[q], acc[i], acc2[i]);
+          for (int i = 0; i < V; ++i) tile[ss_at((c0 + i) * rank + k)] = SECOND && h ? x2[i] : x[i];
+        }
+        __syncthreads();
+        void* dst = h ? out2 : out;
+        const int oes = odp_dtype_size(odt);
+        for (int i = tid * V; i < run; i += SS_THREADS * V) {
+          const int64_t o = m0 * rank + i;
+          if (i + V <= run) {
+            float y[V];
+#pragma unroll
+            for (int q = 0; q < V; ++q) y[q] = tile[ss_at(i) + q];
+            ss_put<V>(dst, o, odt, (((uintptr_t)dst + o * oes) & (V * oes - 1) & 15) == 0, y);
+          } else {
+            for (int q = i; q < run; ++q) odp_store_from_float(dst, m0 * rank + q, odt, tile[ss_at(q)]);
+          }
+        }
+      }
+    }
   }
-  for (; s < n_seg; ++s) {
-    const float c = (float)sc[sex[seg_first + s]];
-    float v[SS_ELEMS];
-    ss_load8_col<BF>(pe, (int64_t)s * E + e_first, M, v);
-#pragma unroll
-    for (int i = 0; i < SS_ELEMS; ++i) ss_term<SECOND, BF>(v[i], c, acc[i], acc2[i]);
-  }
-  float x[SS_ELEMS], x2[SS_ELEMS];
-#pragma unroll
-  for (int i = 0; i < SS_ELEMS; ++i) {
-    x[i] = ss_finish(acc[i], normalize_by, odt);
-    if (SECOND) x2[i] = ss_finish(acc2[i], normalize_by, odt);
-  }
-  ss_put8(out, o, odt, x);
-  if (SECOND) ss_put8(out2, o, odt, x2);
 }
 
 __global__ __launch_bounds__(SS_THREADS) void k_scale_sum(
     const int64_t* __restrict__ probs, const int32_t* __restrict__ ws, int n_prob,
     const int32_t* __restrict__ sex, const double* __restrict__ scales, int n_ex, int n_groups,
     float normalize_by) {
+  __shared__ float tile[SS_THREADS * 8 + SS_THREADS / 4];
   const int bid = blockIdx.x;
   const int p = odp_find_problem(ws, n_prob, bid);
   const int64_t* f = probs + (int64_t)p * ODP_SS_FIELDS;
-  const float* pe = (const float*)f[ODP_SS_PE];
+  const void* pe = (const void*)f[ODP_SS_PE];
   const int64_t M = f[ODP_SS_M];
   const int rank = (int)f[ODP_SS_RANK];
   const int seg_first = (int)f[ODP_SS_SEG_FIRST], n_seg = (int)f[ODP_SS_NSEG];
@@ -398,65 +446,93 @@ __global__ __launch_bounds__(SS_THREADS) void k_scale_sum(
   const int pdt = (int)((flags >> 56) & 0xff);
   const int64_t E = M * rank;
   const double* sc = scales + ((int64_t)cls * n_groups + grp) * n_ex;
-  const bool generic = wide || raw || pdt == ODP_DTYPE_F64 || pdt == ODP_DTYPE_F16 || odt == ODP_DTYPE_F16 ||
-                       odt == ODP_DTYPE_F64 || (E & 7) != 0;
+  const int b = bid - ws[p], nblk = ws[p + 1] - ws[p];
+  const int vec = pdt == ODP_DTYPE_F32 ? 4 : 8;
+  const bool aligned = ((uintptr_t)pe & 15) == 0;
+  // Transposed leaves need whole 16-byte pieces of a row and a tile of at
+  // least one piece per rank; row leaves take any length.
+  const bool fast_t = transpose && aligned && M % vec == 0 && rank <= SS_THREADS;
+  const bool generic = wide || raw || pdt == ODP_DTYPE_F64 || odt == ODP_DTYPE_F64 || (transpose && !fast_t);
   if (generic) {
-    const int64_t e0 = ((int64_t)(bid - ws[p]) * SS_THREADS + threadIdx.x) * SS_ELEMS;
-    if (e0 >= E) return;
-    if (wide || pdt == ODP_DTYPE_F64)
-      scale_sum_generic<double>(pe, pdt, E, e0, n_seg, seg_first, sex, sc, normalize_by, out, out2, odt, transpose,
-                                M, rank, raw);
-    else
-      scale_sum_generic<float>(pe, pdt, E, e0, n_seg, seg_first, sex, sc, normalize_by, out, out2, odt, transpose,
-                               M, rank, raw);
-    return;
-  }
-  const bool bf_in = pdt == ODP_DTYPE_BF16;
-  const int b = bid - ws[p];
-  // Transposed leaves ([M][rank] out of [rank][M] sums) with rank in
-  // {8, 16, 32, 64}: each thread sums 8 consecutive ranks of one column, so
-  // that its outputs are one 16-byte store; lanes take consecutive columns,
-  // so every load instruction reads consecutive elements of a row.
-  const int k8 = rank >> 3;
-  if (transpose && (rank & 7) == 0 && rank <= 64 && SS_THREADS % k8 == 0) {
-    const int cols = SS_THREADS / k8;  // columns per workgroup
-    const int64_t m = (int64_t)b * cols + threadIdx.x % cols;
-    if (m >= M) return;
-    const int64_t e_first = (int64_t)(threadIdx.x / cols) * 8 * M + m;  // element (k0, m)
-    if (out2) {
-      if (bf_in) scale_sum_cols<true, true>(pe, E, M, e_first, n_seg, seg_first, sex, sc, normalize_by, out, out2,
-                                            odt, m * rank + (threadIdx.x / cols) * 8);
-      else scale_sum_cols<true, false>(pe, E, M, e_first, n_seg, seg_first, sex, sc, normalize_by, out, out2, odt,
-                                       m * rank + (threadIdx.x / cols) * 8);
-    } else {
-      if (bf_in) scale_sum_cols<false, true>(pe, E, M, e_first, n_seg, seg_first, sex, sc, normalize_by, out,
-                                             nullptr, odt, m * rank + (threadIdx.x / cols) * 8);
-      else scale_sum_cols<false, false>(pe, E, M, e_first, n_seg, seg_first, sex, sc, normalize_by, out, nullptr,
-                                        odt, m * rank + (threadIdx.x / cols) * 8);
+    for (int64_t e0 = ((int64_t)b * SS_THREADS + threadIdx.x) * SS_ELEMS; e0 < E;
+         e0 += (int64_t)nblk * SS_THREADS * SS_ELEMS) {
+      if (wide || pdt == ODP_DTYPE_F64)
+        scale_sum_generic<double>(pe, pdt, E, e0, n_seg, seg_first, sex, sc, normalize_by, out, out2, odt, transpose,
+                                  M, rank, raw);
+      else
+        scale_sum_generic<float>(pe, pdt, E, e0, n_seg, seg_first, sex, sc, normalize_by, out, out2, odt, transpose,
+                                 M, rank, raw);
     }
     return;
   }
-  const int64_t e0 = ((int64_t)b * SS_THREADS + threadIdx.x) * SS_ELEMS;
-  if (e0 >= E) return;
-  if (out2) {
-    if (bf_in) scale_sum_rows<true, true>(pe, E, M, rank, e0, n_seg, seg_first, sex, sc, normalize_by, out, out2,
-                                          odt, transpose);
-    else scale_sum_rows<true, false>(pe, E, M, rank, e0, n_seg, seg_first, sex, sc, normalize_by, out, out2, odt,
-                                     transpose);
+  const bool rows16 = aligned && E % vec == 0;
+#define ODP_SS_RUN(SECOND, PDT)                                                                                  \
+  do {                                                                                                           \
+    if (transpose || rows16)                                                                                     \
+      scale_sum_fast<SECOND, PDT, true>(pe, M, rank, transpose != 0, b, nblk, n_seg, seg_first, sex, sc,         \
+                                        normalize_by, out, out2, odt, tile);                               \
+    else                                                                                                         \
+      scale_sum_fast<SECOND, PDT, false>(pe, M, rank, false, b, nblk, n_seg, seg_first, sex, sc, normalize_by,   \
+                                         out, out2, odt, tile);                                            \
+  } while (0)
+  if (out2 != nullptr) {
+    if (pdt == ODP_DTYPE_F32) ODP_SS_RUN(true, ODP_DTYPE_F32);
+    else if (pdt == ODP_DTYPE_BF16) ODP_SS_RUN(true, ODP_DTYPE_BF16);
+    else ODP_SS_RUN(true, ODP_DTYPE_F16);
   } else {
-    if (bf_in) scale_sum_rows<false, true>(pe, E, M, rank, e0, n_seg, seg_first, sex, sc, normalize_by, out,
-                                           nullptr, odt, transpose);
-    else scale_sum_rows<false, false>(pe, E, M, rank, e0, n_seg, seg_first, sex, sc, normalize_by, out, nullptr,
-                                      odt, transpose);
+    if (pdt == ODP_DTYPE_F32) ODP_SS_RUN(false, ODP_DTYPE_F32);
+    else if (pdt == ODP_DTYPE_BF16) ODP_SS_RUN(false, ODP_DTYPE_BF16);
+    else ODP_SS_RUN(false, ODP_DTYPE_F16);
   }
+#undef ODP_SS_RUN
 }
 
 // Per-segment sums of squares of materialised per-example tensors: x^2 in
 // clip_pytree's accumulation dtype (float32, or float64 with the flag bit 8
 // of ODP_SQ_DTYPE, as for float64 leaves), summed in fp64.  Each workgroup
-// reduces SQ_CHUNK elements of one segment and writes one slot.
+// reduces SQ_CHUNK elements of one segment and writes one slot.  HBM-bound:
+// 16-byte loads, SQ_DEPTH of them in flight per thread, of the aligned middle
+// of the chunk (a segment's row of n elements may start anywhere), the few
+// elements before and after it one by one.
 constexpr int SQ_THREADS = 256;
 constexpr int64_t SQ_CHUNK = 8192;
+constexpr int SQ_DEPTH = 4;
+
+// One element's square in fp64; non-finite values count as 0 unless `raw`.
+__device__ __forceinline__ double sq_term(float x, bool raw) {
+  if (!raw && !isfinite(x)) x = 0.f;
+  return (double)__fmul_rn(x, x);
+}
+
+template <int PDT>
+__device__ __forceinline__ double sq_chunk(const void* X, int64_t at, int n, bool raw) {
+  constexpr int V = ss_vec<PDT>(), ES = PDT == ODP_DTYPE_F32 ? 4 : 2;
+  const char* p = (const char*)X + at * ES;
+  int head = (int)((16 - ((uintptr_t)p & 15)) & 15) / ES;
+  head = head < n ? head : n;
+  const int pieces = (n - head) / V, tail = head + pieces * V;
+  const ODP_GMEM ss_u32x4* v = (const ODP_GMEM ss_u32x4*)(const ODP_GMEM void*)(p + head * ES);
+  double a = 0.0, b = 0.0;
+  if ((int)threadIdx.x < head) a = sq_term(odp_load_as_float(X, at + threadIdx.x, PDT), raw);
+  if (tail + (int)threadIdx.x < n) b = sq_term(odp_load_as_float(X, at + tail + threadIdx.x, PDT), raw);
+  for (int i0 = threadIdx.x; i0 < pieces; i0 += SQ_DEPTH * SQ_THREADS) {
+    ss_u32x4 w[SQ_DEPTH];
+#pragma unroll
+    for (int q = 0; q < SQ_DEPTH; ++q) w[q] = i0 + q * SQ_THREADS < pieces ? v[i0 + q * SQ_THREADS] : ss_u32x4{0u, 0u, 0u, 0u};
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < SQ_DEPTH; ++q) {
+      float x[V];
+      ss_unpack<PDT>(w[q], x);
+#pragma unroll
+      for (int i = 0; i < V; i += 2) {
+        a += sq_term(x[i], raw);
+        b += sq_term(x[i + 1], raw);
+      }
+    }
+  }
+  return a + b;
+}
 
 // Writes outside the partials ([0, n_ex) x [0, part_stride)) are dropped;
 // `status` (optional) is then set to 1.
@@ -475,9 +551,9 @@ __global__ __launch_bounds__(SQ_THREADS) void k_sqnorm(const int64_t* __restrict
   const int dt = (int)(f[ODP_SQ_DTYPE] & 0xff);
   const bool sq64 = ((f[ODP_SQ_DTYPE] >> 8) & 1) != 0;
   const bool raw = ((f[ODP_SQ_DTYPE] >> 9) & 1) != 0;  // no nan_to_num
-  const int64_t nchunk = (n + SQ_CHUNK - 1) / SQ_CHUNK;
-  const int64_t local = bid - ws[p];
-  const int64_t seg = local / nchunk, chunk = local % nchunk;
+  const int nchunk = (int)((n + SQ_CHUNK - 1) / SQ_CHUNK);
+  const int local = bid - ws[p];
+  const int seg = local / nchunk, chunk = local - seg * nchunk;
   const int64_t lo = chunk * SQ_CHUNK, hi = lo + SQ_CHUNK < n ? lo + SQ_CHUNK : n;
   double acc = 0.0;
   if (sq64) {
@@ -486,24 +562,25 @@ __global__ __launch_bounds__(SQ_THREADS) void k_sqnorm(const int64_t* __restrict
       if (!raw && !isfinite(x)) x = 0.0;  // nan_to_num before the norm
       acc += x * x;
     }
+  } else if (dt == ODP_DTYPE_F32) {
+    acc = sq_chunk<ODP_DTYPE_F32>(X, seg * n + lo, (int)(hi - lo), raw);
+  } else if (dt == ODP_DTYPE_BF16) {
+    acc = sq_chunk<ODP_DTYPE_BF16>(X, seg * n + lo, (int)(hi - lo), raw);
+  } else if (dt == ODP_DTYPE_F16) {
+    acc = sq_chunk<ODP_DTYPE_F16>(X, seg * n + lo, (int)(hi - lo), raw);
   } else {
-    for (int64_t i = lo + threadIdx.x; i < hi; i += SQ_THREADS) {
-      float x = odp_load_as_float(X, seg * n + i, dt);
-      if (!raw && !isfinite(x)) x = 0.f;
-      acc += (double)__fmul_rn(x, x);
-    }
+    for (int64_t i = lo + threadIdx.x; i < hi; i += SQ_THREADS)
+      acc += sq_term(odp_load_as_float(X, seg * n + i, dt), raw);
   }
-  __shared__ double red[SQ_THREADS];
-  red[threadIdx.x] = acc;
+  __shared__ double red[SQ_THREADS / 64];
+  acc = rows_sum4(row_sum16(acc));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
   __syncthreads();
-  for (int w = SQ_THREADS / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] = red[threadIdx.x] + red[threadIdx.x + w];
-    __syncthreads();
-  }
   if (threadIdx.x == 0) {
+    const double tot = (red[0] + red[1]) + (red[2] + red[3]);
     const int ex = sex[seg_first + seg];
     if (ex >= 0 && ex < n_ex && slot >= 0 && slot + chunk < part_stride)
-      part[(int64_t)ex * part_stride + slot + chunk] = red[0];
+      part[(int64_t)ex * part_stride + slot + chunk] = tot;
     else if (status != nullptr)
       odp_gstore(status, 1u);  // every such writer stores the same value
   }
@@ -587,7 +664,7 @@ extern "C" int odp_clip_factors(odp_stream_t stream, const double* part, int64_t
 }
 
 extern "C" int64_t odp_scale_sum_blocks(int64_t n_elems) {
-  const int64_t per = (int64_t)SS_THREADS * SS_ELEMS;
+  const int64_t per = (int64_t)SS_THREADS * 8;  // a tile of 16-bit values
   return n_elems <= 0 ? 0 : (n_elems + per - 1) / per;
 }
 

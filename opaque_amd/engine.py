@@ -534,8 +534,9 @@ _STREAM_STAGES = ("factor_stream", "factor_stream_long")
 # are split into smaller column groups than odp_seg_factor_stream_groups()'s.
 STREAM_SLOTS_PER_CU = 2
 STREAM_ROUNDS = 4
+STREAM_MIN_ROUNDS = 1
 # Steps (64 tokens of one 256-column tile) a column group should at least hold.
-STREAM_MIN_STEPS = 8
+STREAM_MIN_STEPS = 10
 
 # Stages launched after the clip factors, in table order.
 _AFTER_CLIP = ("scale_sum", "lin_prescale", "lin_sum", "lin_moments")
@@ -1267,7 +1268,7 @@ class GhostPlan:
                     N.SS_PE: pe_a, N.SS_M: M, N.SS_RANK: rank, N.SS_SEG_FIRST: v.first,
                     N.SS_NSEG: n_seg, N.SS_OUT: out.data_ptr(), N.SS_FLAGS: flags, N.SS_OUT2: out2,
                 },
-                lib.odp_scale_sum_blocks(rank * M),
+                lib.odp_scale_sum_blocks(rank * M) * self._sum_split(rank * M, pdt),
                 n_seg * rank * M * (self.pe[pe_dt[i]].element_size() if i not in mat_pe else mat_pe[i].element_size())
                 + rank * M * out.element_size() * (2 if self.out2 is not None else 1),
                 io=rank * M * out.element_size() * (2 if self.out2 is not None else 1),
@@ -1774,19 +1775,20 @@ class GhostPlan:
         """The streamed rows as one table per rank block count, most work per
         workgroup first.  A segment's 256-column tiles go to groups of
         odp_seg_factor_stream_groups()'s size; while the launch would not
-        fill the chip STREAM_ROUNDS times, to smaller ones of at least
-        STREAM_MIN_STEPS steps."""
+        fill the chip STREAM_ROUNDS times, to smaller ones, of at least
+        STREAM_MIN_STEPS steps where that still fills it STREAM_MIN_ROUNDS
+        times."""
         lib = N.load()
         slots = STREAM_SLOTS_PER_CU * torch.cuda.get_device_properties(self.device).multi_processor_count \
             if self.device.type == "cuda" else 1
         tiles = sum((M + 255) // 256 * int((ln > 0).sum()) for lst in rows.values() for _, ln, M, *_ in lst)
-        per = max(1, tiles // (STREAM_ROUNDS * slots))
+        per, most = max(1, tiles // (STREAM_ROUNDS * slots)), max(1, tiles // (STREAM_MIN_ROUNDS * slots))
         out: dict[int, _Table] = {}
         for nkb in sorted(rows):
             work = []
             for arr, ln, M, *_ in rows[nkb]:
                 n = (M + 255) // 256
-                size = np.maximum(per, -(-STREAM_MIN_STEPS // np.maximum((ln + 63) // 64, 1)))
+                size = np.maximum(per, np.minimum(most, -(-STREAM_MIN_STEPS // np.maximum((ln + 63) // 64, 1))))
                 arr[:, N.FT_GROUPS] = np.maximum(int(lib.odp_seg_factor_stream_groups(M)), -(-n // size))
                 work.append(ln * M / arr[:, N.FT_GROUPS])
             order = np.argsort(-np.concatenate(work), kind="stable")
@@ -1806,6 +1808,14 @@ class GhostPlan:
             row[N.FT_LEAF0 + 3 * li + 1] = (c - col0) | (rk << 16) | self._pe_bits(leaf)
             row[N.FT_LEAF0 + 3 * li + 2] = slot_base[leaf]
         return row
+
+    @staticmethod
+    def _sum_split(n: int, pdt: int) -> int:
+        """Workgroups per 2048 elements of a clipped sum, one tile each: float32
+        and float64 values take 4 elements a thread, 16-bit ones 8, rows of a
+        length off the 16-byte grid one."""
+        vec = 4 if pdt in (N.DTYPE_F32, N.DTYPE_F64) else 8
+        return 8 // vec if n % vec == 0 else 8
 
     def _leaf_transposed(self, i: int, sites: list[LoraSite]) -> bool:
         # pe rows are [r][M]; A leaves [d_in, r] need the transpose, B leaves [r, d_out] do not.

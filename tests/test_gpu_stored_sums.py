@@ -1,0 +1,144 @@
+"""Norms and clipped sums of stored per-example gradients, at the edges of
+their vector paths.
+
+odp_sqnorm reads 16-byte pieces of each example's row and the elements before
+and after them one by one, odp_scale_sum takes rows in 16-byte pieces, rows of
+other lengths element by element, and transposed LoRA leaves through LDS
+tiles of whole columns, and odp_clip_factors sums several groups side by side.
+
+The clipped sum is defined to the bit (clip_pytree's scale.to(dtype) * leaf
+rounded to the leaf's dtype, a float32 sum over the examples in order, a cast
+and a division in the output dtype), so it is compared with those torch
+operations exactly for 16-bit values.  For float32 ones the kernel adds
+scale * value by fused multiply-adds, which leave out the product's rounding:
+each term may differ by half a unit in its last place, and each partial sum
+rounds differently in turn, within sqrt(n) 2^-23 of the sum of magnitudes.  Norms are fp64 sums of float32 squares in some order,
+returned in float32: rel 1e-6.
+"""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from opaque_amd import _native as N
+from opaque_amd.engine import ClipSpec, GhostPlan, LeafOut, LoraSite, MaterializedLeaf, Segments
+from opaque_amd.guard import guard_constants, leaf_guards
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _clip(leaves, dtype, thresholds):
+    _, rnd = leaf_guards([lf.shape for lf in leaves], [dtype] * len(leaves))
+    rel, ab = guard_constants(dtype, rnd)
+    return ClipSpec(mode=N.CLIP_FIXED, thresholds=thresholds, effective=math.sqrt(sum(t * t for t in thresholds)),
+                    normalize_by=3.0, guards=[(rel, ab, dtype)])
+
+
+def _close(got, want, pe, c, power=1):
+    if pe.dtype != torch.float32:
+        return torch.equal(got, want)
+    v = torch.where(torch.isfinite(pe), pe, torch.zeros_like(pe)).double()
+    mag = (c.view(-1, *[1] * (pe.dim() - 1)) * v).abs().pow(power).sum(0)
+    return bool(((got.double() - want.double()).abs() <= 2.0**-23 * pe.shape[0] ** 0.5 * mag).all())
+
+
+def _sums(pe, c, out_dtype, nb=3.0):
+    """Clipped sum and second moment of pe [n, ...] with scales c [n], torch operation by operation on the
+    host (IEEE division)."""
+    pe, c = pe.cpu(), c.cpu()
+    acc = acc2 = torch.zeros(pe.shape[1:], dtype=torch.float32)
+    v = torch.where(torch.isfinite(pe), pe, torch.zeros_like(pe))
+    for i in range(pe.shape[0]):
+        y = c[i].to(pe.dtype) * v[i]
+        acc = acc + y.float()
+        acc2 = acc2 + (y * y).float()
+    return [(t.to(out_dtype) / torch.tensor(nb, dtype=out_dtype)).to(DEV) for t in (acc, acc2)]
+
+
+# (elements per example, examples): below, at and past one piece, one workgroup's tile and one chunk of
+# the norm kernel; odd rows; several groups of segments and a rest.
+ROWS = [(1, 1), (3, 5), (8, 9), (1001, 17), (1024, 8), (2048, 4), (2052, 3), (8191, 2), (8192, 7), (24580, 13)]
+
+
+@pytest.mark.parametrize("second", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,n_ex", ROWS)
+def test_materialised_rows(n, n_ex, dtype, second):
+    print(f"stored sums: {n} x {n_ex} {dtype} second={second}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(n + n_ex)
+    spread = torch.logspace(-1, 1, n_ex, device=DEV).view(-1, 1)
+    # One element past the allocation's start: rows off the 16-byte grid where the dtype and length allow it.
+    pe = (torch.randn(n_ex * n + 1, device=DEV, generator=g)[1:].view(n_ex, n) * spread).to(dtype)
+    pe[0, 0] = float("nan")
+    pe[n_ex - 1, n - 1] = float("-inf")
+    leaves = [LeafOut((n,), dtype)]
+    finite = torch.where(torch.isfinite(pe), pe, torch.zeros_like(pe)).float()
+    norms = finite.square().double().sum(1).sqrt()
+    C = float(norms.median())
+    plan = GhostPlan(segments=Segments.padded(n_ex, 1), leaves=leaves, clip=_clip(leaves, dtype, [C]),
+                     materialized=[MaterializedLeaf(pe, 0)], device=DEV, second_moment=second)
+    res = plan.run()
+    torch.cuda.synchronize()
+    assert torch.allclose(res.norms.double(), norms, rtol=1e-6, atol=0)
+    want = _sums(pe, res.scales[0, 0], dtype)
+    assert _close(res.leaves[0], want[0], pe, res.scales[0, 0])
+    if second:
+        assert _close(res.second_moment[0], want[1], pe, res.scales[0, 0], 2)
+
+
+@pytest.mark.parametrize("second", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("r", [1, 4, 8, 12, 20, 64])
+def test_transposed_leaves(r, dtype, second):
+    """A leaf [d_in, r] and B leaf [d_out, r], both transposed from the [r][M]
+    rows the plan stores; widths of less than one tile and of several with a
+    rest."""
+    print(f"stored sums: transposed rank {r} {dtype} second={second}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(r)
+    n_ex, T, d_in, d_out = 9, 8, 24, 2072
+
+    def rnd(*s):
+        return torch.randn(*s, device=DEV, generator=g).to(dtype)
+
+    x, gt, A, B = rnd(n_ex * T, d_in), rnd(n_ex * T, d_out), rnd(d_in, r), rnd(r, d_out)
+    leaves = [LeafOut((d_in, r), dtype), LeafOut((d_out, r), dtype)]
+    site = LoraSite(x, gt, A, B, 0.5, a_leaf=0, b_leaf=1, a_transposed=False, b_transposed=True, v=x @ A,
+                    u=gt @ B.t().contiguous())
+    plan = GhostPlan(segments=Segments.padded(n_ex, T), leaves=leaves, clip=_clip(leaves, dtype, [50.0]),
+                     lora_sites=[site], device=DEV, second_moment=second)
+    res = plan.run()
+    torch.cuda.synchronize()
+    for k, (pe, m) in enumerate(zip(plan.pe_views(), (d_in, d_out))):
+        rows, c = pe.view(n_ex, r, m).transpose(1, 2), res.scales[0, 0]
+        want = _sums(rows, c, dtype)
+        assert _close(res.leaves[k], want[0], rows, c), k
+        if second:
+            assert _close(res.second_moment[k], want[1], rows, c, 2), k
+
+
+@pytest.mark.parametrize("groups", [1, 2, 3, 8, 9, 16, 17, 40])
+def test_groups_side_by_side(groups):
+    """Groups share the clip kernel's 16 waves evenly, one wave each past 8 groups, in rounds past 16."""
+    print(f"stored sums: {groups} clip groups", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(groups)
+    n_ex = 3
+    sizes = [1 + (7919 * k) % 30011 for k in range(groups + 2)]  # one to four partial slots each
+    group = [k % groups for k in range(groups + 2)]
+    pes = [torch.randn(n_ex, n, device=DEV, generator=g) for n in sizes]
+    leaves = [LeafOut((n,), torch.float32, group=k) for n, k in zip(sizes, group)]
+    want = torch.zeros(groups, n_ex, dtype=torch.float64, device=DEV)
+    for pe, k in zip(pes, group):
+        want[k] += pe.square().double().sum(1)
+    C = (want.sqrt().mean(1) * 1.0).tolist()
+    plan = GhostPlan(segments=Segments.padded(n_ex, 1), leaves=leaves, clip=_clip(leaves, torch.float32, C),
+                     materialized=[MaterializedLeaf(pe, k) for k, pe in enumerate(pes)], device=DEV)
+    res = plan.run()
+    torch.cuda.synchronize()
+    assert torch.allclose(res.group_norms.double(), want.sqrt(), rtol=1e-6)
+    assert torch.allclose(res.norms.double(), want.sum(0).sqrt(), rtol=1e-6)
+    thr = torch.tensor(C, device=DEV).view(-1, 1)
+    assert torch.equal(res.clipped.bool(), res.group_norms > thr.float())
