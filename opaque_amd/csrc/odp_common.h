@@ -9,23 +9,22 @@
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-// Round-to-nearest-even float -> bf16 bit pattern (NaN stays NaN).
-__device__ __forceinline__ uint16_t odp_f2bf(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
+// Round-to-nearest-even float -> bf16 bit pattern by the hardware conversion
+// (v_cvt_pk_bf16_f32; NaN stays NaN).
+__device__ __forceinline__ uint16_t odp_f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
+// Two of them: lo in the low half.
+__device__ __forceinline__ uint32_t odp_f2bf2(float lo, float hi) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
 
 __device__ __forceinline__ float odp_bf2f(uint16_t h) {
   return __uint_as_float(((uint32_t)h) << 16);
 }
 
-// A finite float rounded to nearest-even bfloat16, by the hardware
-// conversion (v_cvt_pk_bf16_f32).
-__device__ __forceinline__ float odp_round_bf16(float f) {
-  return odp_bf2f(__builtin_bit_cast(uint16_t, (__bf16)f));
-}
+// A float rounded to nearest-even bfloat16.
+__device__ __forceinline__ float odp_round_bf16(float f) { return odp_bf2f(odp_f2bf(f)); }
 
 // s_waitcnt immediate: vmcnt <= n (0..63), lgkmcnt and expcnt not waited on.
 __host__ __device__ constexpr uint32_t vmcnt_imm(int n) {

@@ -197,7 +197,7 @@ __device__ __forceinline__ void factor_epilogue(const f32x4_t (&acc)[NJ][NKB], i
                                                 int ex, int64_t part_stride,
                                                 const FactorLeaves& L, double* __restrict__ part) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  double wsum[4] = {0.0, 0.0, 0.0, 0.0};  // this wave's sum of squares per leaf
+  double lsum[4] = {0.0, 0.0, 0.0, 0.0};  // this lane's sum of squares per leaf
 #pragma unroll
   for (int kb = 0; kb < NKB; ++kb) {
     double cs[4];
@@ -269,23 +269,21 @@ __device__ __forceinline__ void factor_epilogue(const f32x4_t (&acc)[NJ][NKB], i
         odp_gstore((u32x4_t*)(lpe + at), u32x4_t{x[0], x[1], x[2], x[3]});
       }
     }
-    // Sum over the 16 lanes that share a column (same lane >> 4), then add
-    // the column to its leaf's sum.
+    // Each column's squares to its leaf's sum.
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const double v = row_sum16(cs[i]);
       const int k = kb * 16 + 4 * (lane >> 4) + i;
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        if (q < L.n && k >= L.col0[q] && k < L.col0[q] + L.rank[q]) wsum[q] += v;
+        if (q < L.n && k >= L.col0[q] && k < L.col0[q] + L.rank[q]) lsum[q] += cs[i];
     }
   }
-  // The four column groups of the wave, then one slot per (tile, wave): no
-  // workgroup barrier, and a fixed order, so runs stay bitwise reproducible.
+  // The lanes of the wave, then one slot per (tile, wave): no workgroup
+  // barrier, and a fixed order, so runs stay bitwise reproducible.
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     if (q < L.n) {
-      const double v = rows_sum4(wsum[q]);
+      const double v = rows_sum4(row_sum16(lsum[q]));
       if (lane == 0) odp_gstore(part + (int64_t)ex * part_stride + L.slot[q] + ODP_FT_WAVE_SLOTS * tile + wave, v);
     }
   }
@@ -672,7 +670,7 @@ __device__ __forceinline__ void factor_pass_bf16(const int64_t* __restrict__ f, 
   auto emit = [&](const f32x4_t (&acc)[NJ][NKB], bool live, int32_t m_base, int tile) __attribute__((always_inline)) {
     const int t = lane & 3, tl = t & 1, th = t >> 1;
     const int kt = 4 * (lane >> 4) + t;
-    double wsum = 0.0;
+    double lsum = 0.0;
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb) {
       const int rk = lrank[kb];
@@ -681,26 +679,27 @@ __device__ __forceinline__ void factor_pass_bf16(const int64_t* __restrict__ f, 
       const __amdgpu_buffer_rsrc_t part_rsrc = __builtin_amdgcn_make_buffer_rsrc(
           (void*)(part + (int64_t)ex * part_stride + lslot[kb]), (short)0,
           llast[kb] ? (int)(ODP_FT_WAVE_SLOTS * (uint32_t)nchunks * 8u) : 0, ODP_BUFFER_DWORD3);
+      // Rows past the leaf's (and whole blocks without one) hold whatever
+      // their plane rows made of P; columns past M are zero.
       double cs[4] = {0.0, 0.0, 0.0, 0.0};
-      if (!lcont[kb]) wsum = 0.0;
+      if (!lcont[kb]) lsum = 0.0;
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        const int32_t m = m_base + (NJ * wave + j) * 16 + (lane & 15);
-        uint32_t h[4];
+        // Rows 4g, 4g + 1 and 4g + 2, 4g + 3 of the lane's column, as stored.
+        const uint32_t h01 = odp_f2bf2(scale * acc[j][kb][0], scale * acc[j][kb][1]);
+        const uint32_t h23 = odp_f2bf2(scale * acc[j][kb][2], scale * acc[j][kb][3]);
+        const float vq[4] = {__uint_as_float(h01 << 16), __uint_as_float(h01 & 0xffff0000u),
+                             __uint_as_float(h23 << 16), __uint_as_float(h23 & 0xffff0000u)};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          h[i] = odp_f2bf(scale * acc[j][kb][i]);
-          if (4 * (lane >> 4) + i < rk && m < M) {
-            const float vq = odp_bf2f((uint16_t)h[i]);  // the value as stored
-            const float vf = isfinite(vq) ? vq : 0.f;
-            cs[i] += (double)__fmul_rn(vf, vf);
-          }
+          const float vf = isfinite(vq[i]) && 4 * (lane >> 4) + i < rk ? vq[i] : 0.f;
+          cs[i] += (double)__fmul_rn(vf, vf);
         }
         // Rows of the other parity to the odd/even neighbour.
-        const uint32_t r1 = quad_x1(tl ? (h[0] | (h[2] << 16)) : (h[1] | (h[3] << 16)));
+        const uint32_t r1 = quad_x1(tl ? ((h01 & 0xffffu) | (h23 << 16)) : ((h01 >> 16) | (h23 & 0xffff0000u)));
         // Rows 4g + 2a + tl, columns of this lane pair (low half: even column).
-        const uint32_t p0 = tl ? ((r1 & 0xffffu) | (h[1] << 16)) : (h[0] | (r1 << 16));
-        const uint32_t p1 = tl ? ((r1 >> 16) | (h[3] << 16)) : (h[2] | (r1 & 0xffff0000u));
+        const uint32_t p0 = tl ? ((r1 & 0xffffu) | (h01 & 0xffff0000u)) : ((h01 & 0xffffu) | (r1 << 16));
+        const uint32_t p1 = tl ? ((r1 >> 16) | (h23 & 0xffff0000u)) : ((h23 & 0xffffu) | (r1 & 0xffff0000u));
         // Row pairs across the two lane pairs of the quad.
         const uint32_t r2 = quad_x2(th ? p0 : p1);
         const uint32_t keep = th ? p1 : p0;
@@ -709,11 +708,8 @@ __device__ __forceinline__ void factor_pass_bf16(const int64_t* __restrict__ f, 
         __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{th ? r2 : keep, th ? keep : r2}, pe_rsrc, (int)off, 0, 0);
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const double v = row_sum16(cs[i]);
-        if (4 * (lane >> 4) + i < rk) wsum += v;
-      }
-      const double sq = rows_sum4(wsum);
+      for (int i = 0; i < 4; ++i) lsum += cs[i];
+      const double sq = llast[kb] ? rows_sum4(row_sum16(lsum)) : 0.0;
       const uint32_t poff =
           live && lane == 0 ? (uint32_t)(ODP_FT_WAVE_SLOTS * tile + wave) * 8u : 0x80000000u;
       __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, sq), part_rsrc, (int)poff, 0, 0);
