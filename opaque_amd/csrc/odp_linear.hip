@@ -56,6 +56,16 @@ __device__ __forceinline__ bool seg_item(int local, int n_seg, int per_seg, int&
   return seg < n_seg;
 }
 
+// Tile t of the work order of a tm x tn tile grid: groups of OUTER_GROUP tile
+// rows, each walked column by column, so that consecutive tiles (which one
+// XCD computes at a time) share operand columns: 32 tiles read 8 blocks of G
+// and 4 of X.
+__device__ __forceinline__ int grouped_tile(int t, int tm, int tn) {
+  const int per_group = OUTER_GROUP * tn, g = t / per_group, first = g * OUTER_GROUP;
+  const int gm = min(tm - first, OUTER_GROUP), r = t - g * per_group;
+  return (first + r % gm) * tn + r / gm;
+}
+
 // Block-wide fp64 sum; the result is valid in thread 0.
 __device__ __forceinline__ double block_sum(double v, double* red) {
 #pragma unroll
@@ -71,11 +81,34 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
   return t;
 }
 
-// fp32 squares of the finite entries, summed in fp64; `nonfinite` is set
-// when an entry was not finite (and counted as 0).
+// Squares of the finite entries, summed in fp64; `nonfinite` is set when an
+// entry was not finite (and counted as 0).  A float32 sum of squares over the
+// wave's entries tells the usual case, nothing non-finite and no square past
+// float32's range, in one instruction an entry; the squares are then exact in
+// fp64.  Otherwise each is a float32 square, infinite where it overflows, as
+// the reference's float32 accumulation dtype has it.
 template <int I, int J>
 __device__ __forceinline__ double acc_sq(const f32x4_t (&acc)[I][J], bool& nonfinite) {
-  double s = 0.0;
+  float c[4] = {0.f, 0.f, 0.f, 0.f};
+  static_for<I * J>([&](auto q) {
+    constexpr int i = decltype(q)::value / J, j = decltype(q)::value % J;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c[e] = __builtin_fmaf(acc[i][j][e], acc[i][j][e], c[e]);
+  });
+  double s[2] = {0.0, 0.0};
+  if (__builtin_amdgcn_ballot_w64(!isfinite((c[0] + c[1]) + (c[2] + c[3]))) == 0) {
+    static_for<I * J>([&](auto q) {
+      constexpr int i = decltype(q)::value / J, j = decltype(q)::value % J;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const double v = (double)acc[i][j][e];
+        s[e & 1] = __builtin_fma(v, v, s[e & 1]);
+      }
+      // One tile's accumulators at a time in fp64.
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    return s[0] + s[1];
+  }
   static_for<I * J>([&](auto q) {
     constexpr int i = decltype(q)::value / J, j = decltype(q)::value % J;
 #pragma unroll
@@ -84,12 +117,11 @@ __device__ __forceinline__ double acc_sq(const f32x4_t (&acc)[I][J], bool& nonfi
       const bool fin = isfinite(v);
       nonfinite |= !fin;
       const float vf = fin ? v : 0.f;
-      s += (double)__fmul_rn(vf, vf);
+      s[0] += (double)__fmul_rn(vf, vf);
     }
-    // One tile's accumulators at a time in VGPRs.
     __builtin_amdgcn_sched_barrier(0);
   });
-  return s;
+  return s[0];
 }
 
 // ---------------------------------------------------------------------------
@@ -101,7 +133,7 @@ __global__ __launch_bounds__(OUTER_THREADS, ODP_LIN_OCC) void k_lin_outer_norm(c
                                                         const int32_t* __restrict__ slen,
                                                         const int32_t* __restrict__ sex,
                                                         double* __restrict__ part, int64_t part_stride) {
-  __shared__ double red[NW];
+  double* red = (double*)lin_ring4;  // a stage the store of M_s does not use
   const int bid = blockIdx.x;
   const int p = odp_find_problem(ws, n_prob, bid);
   const int64_t* f = probs + (int64_t)p * ODP_LN_FIELDS;
@@ -119,13 +151,7 @@ __global__ __launch_bounds__(OUTER_THREADS, ODP_LIN_OCC) void k_lin_outer_norm(c
   const int pid = (local & 7) * (nblk >> 3) + (local >> 3);
   if (pid >= P.n_seg * tiles) return;
   const int seg = pid / tiles;
-  int tile;
-  {
-    const int t = pid - seg * tiles;
-    const int per_group = OUTER_GROUP * tn_count, g = t / per_group, first_m = g * OUTER_GROUP;
-    const int gm = min(tm_count - first_m, OUTER_GROUP), rr = t - g * per_group;
-    tile = (first_m + rr % gm) * tn_count + rr / gm;
-  }
+  const int tile = grouped_tile(pid - seg * tiles, tm_count, tn_count);
   const int64_t o0 = (int64_t)(tile / tn_count) * OM, n0 = (int64_t)(tile % tn_count) * ON;
   const int gs = P.seg_first + seg;
   const int64_t t_begin = sstart[gs], t_end = t_begin + slen[gs];
@@ -140,7 +166,7 @@ __global__ __launch_bounds__(OUTER_THREADS, ODP_LIN_OCC) void k_lin_outer_norm(c
     n.live = n.t0 < st.te ? 1 : 0;
     return n;
   };
-  dma_mainloop<false, true, false>(P, o0, n0, first, next, [](const Step&) { return 1.0f; },
+  dma_mainloop<false, false>(P, o0, n0, first, next, [](const Step&) { return 1.0f; },
                                    [](uint16_t*, const Step&) {}, acc);
   // Columns/rows past the matrix were zero operands, so they add nothing.
   // Non-finite entries of M_s count 0 (nan_to_num before the norm).
@@ -153,20 +179,18 @@ __global__ __launch_bounds__(OUTER_THREADS, ODP_LIN_OCC) void k_lin_outer_norm(c
   // Optionally keep the tile of M_s itself, rounded to bf16, for a later
   // clipped sum over stored per-example gradients.  Each wave's WM x WN
   // block goes through its own part of the (now idle) LDS ring so that rows
-  // leave in 16-byte pieces: 8-column chunk q of block row r sits at chunk
-  // q ^ ((r >> 2) & 7), which keeps both the 2-byte writes of the MFMA
-  // layout and the 16-byte reads free of bank conflicts.
+  // leave in 16-byte pieces, a whole 128-byte line each: 16-byte piece q of
+  // block row r sits at piece q ^ (r & 7), which keeps both the 8-byte writes
+  // of the MFMA layout and the 16-byte reads free of bank conflicts.
   uint16_t* pe = (uint16_t*)f[ODP_LN_PE];
   if (pe != nullptr) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     uint16_t* stg = lin_stage(wave >> 1) + (wave & 1) * (WM * WN);
     static_for<BI * BJ>([&](auto q) {
       constexpr int i = decltype(q)::value / BJ, j = decltype(q)::value % BJ;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int r = 16 * i + 4 * (lane >> 4) + e, c = 16 * j + (lane & 15);
-        stg[r * WN + 8 * ((c >> 3) ^ ((r >> 2) & 7)) + (c & 7)] = odp_f2bf(acc[i][j][e]);
-      }
+      const int r = acc_row(i), c = acc_col(j);
+      *(u32x2_alias_t*)&stg[r * WN + 8 * ((c >> 3) ^ (r & 7)) + (c & 7)] =
+          u32x2_t{odp_f2bf2(acc[i][j][0], acc[i][j][1]), odp_f2bf2(acc[i][j][2], acc[i][j][3])};
       __builtin_amdgcn_sched_barrier(0);
     });
     uint16_t* dst = pe + (int64_t)seg * P.d_out * P.d_in;
@@ -174,7 +198,7 @@ __global__ __launch_bounds__(OUTER_THREADS, ODP_LIN_OCC) void k_lin_outer_norm(c
 #pragma unroll
     for (int k = 0; k < WM / 8; ++k) {
       const int r = 8 * k + (lane >> 3), qq = lane & 7;
-      const u32x4_t v = *(const u32x4_alias_t*)&stg[r * WN + 8 * (qq ^ ((r >> 2) & 7))];
+      const u32x4_t v = *(const u32x4_alias_t*)&stg[r * WN + 8 * (qq ^ (r & 7))];
       const int64_t o = ob + r, n = nb + 8 * qq;
       // Non-temporal: the stored gradients are read again only by a later
       // launch, and should not evict this launch's operands from L2.
@@ -197,7 +221,7 @@ __global__ __launch_bounds__(OUTER_THREADS, ODP_LIN_OCC) void k_lin_outer_norm_g
     const int64_t* __restrict__ probs, const int32_t* __restrict__ ws, int n_prob,
     const int32_t* __restrict__ sstart, const int32_t* __restrict__ slen, const int32_t* __restrict__ sex,
     double* __restrict__ part, int64_t part_stride) {
-  __shared__ double red[NW];
+  double* red = (double*)lin_ring4;  // a stage the store of M_s does not use
   const int bid = blockIdx.x;
   const int p = odp_find_problem(ws, n_prob, bid);
   const int64_t* f = probs + (int64_t)p * ODP_LN_FIELDS;
@@ -224,7 +248,7 @@ __global__ __launch_bounds__(OUTER_THREADS, ODP_LIN_OCC) void k_lin_outer_norm_g
     OuterAcc acc;
     zero_acc(acc);
     const Step first = {t_begin, t_begin, t_begin + len, seg, 1, 0};
-    dma_mainloop<false, true, false>(P, o0, n0, first, next, [](const Step&) { return 1.0f; },
+    dma_mainloop<false, false>(P, o0, n0, first, next, [](const Step&) { return 1.0f; },
                                      [](uint16_t*, const Step&) {}, acc);
     bool nonfinite = false;
     const double tot = block_sum(acc_sq(acc, nonfinite), red);
@@ -882,22 +906,32 @@ __global__ __launch_bounds__(OUTER_THREADS, ODP_LIN_OCC) void k_lin_clip_sum(con
   const ODP_CONST double* csc = (const ODP_CONST double*)sc;
   auto scale = [&](const Step& st) { return (float)csc[cex[st.seg]]; };
   // PRESCALED: X already holds c_i x_t (odp_linear_prescale).
-  dma_mainloop<!PRESCALED, true, true>(P, o0, n0, at_segment(0), next, scale, fixup, acc);
+  dma_mainloop<!PRESCALED, true>(P, o0, n0, at_segment(0), next, scale, fixup, acc);
 
-  // Lane holds D[4 (lane >> 4) + e][lane & 15] of each 16 x 16 block.
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // 4 consecutive elements of an output row per block: one 8- or 16-byte
+  // store (d_in is a multiple of 8; an output leaf of a stack may start at
+  // any element).
+  const int wave = threadIdx.x >> 6;
   const int wm = WM * (wave & 1), wn = WN * (wave >> 1);
+  const bool vec = ((uintptr_t)out & 15) == 0;
   static_for<BI * BJ>([&](auto q) {
     constexpr int i = decltype(q)::value / BJ, j = decltype(q)::value % BJ;
+    const int64_t o = o0 + wm + acc_row(i), n = n0 + wn + acc_col(j);
+    if (o < P.d_out && n < P.d_in) {
+      float y[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int64_t o = o0 + wm + 16 * i + 4 * (lane >> 4) + e;
-      const int64_t n = n0 + wn + 16 * j + (lane & 15);
-      if (o < P.d_out && n < P.d_in) {
-        float x = odp_round_to(acc[i][j][e], odt);
-        if (normalize_by != 1.0f) x = odp_round_to(__fdiv_rn(x, normalize_by), odt);
-        odp_store_from_float(out, o * P.d_in + n, odt, x);
+      for (int e = 0; e < 4; ++e) {
+        y[e] = odp_round_to(acc[i][j][e], odt);
+        if (normalize_by != 1.0f) y[e] = odp_round_to(__fdiv_rn(y[e], normalize_by), odt);
       }
+      const int64_t at = o * P.d_in + n;
+      if (vec && odt == ODP_DTYPE_BF16)
+        odp_gstore((u32x2_t*)((uint16_t*)out + at), u32x2_t{odp_f2bf2(y[0], y[1]), odp_f2bf2(y[2], y[3])});
+      else if (vec && odt == ODP_DTYPE_F32)
+        odp_gstore((f32x4_t*)((float*)out + at), f32x4_t{y[0], y[1], y[2], y[3]});
+      else
+#pragma unroll
+        for (int e = 0; e < 4; ++e) odp_store_from_float(out, at + e, odt, y[e]);
     }
     // One tile's accumulators at a time in VGPRs.
     __builtin_amdgcn_sched_barrier(0);

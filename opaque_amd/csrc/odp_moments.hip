@@ -84,7 +84,7 @@ __device__ __forceinline__ void moments_tile(const int64_t* __restrict__ f, cons
     if (len <= 0) continue;  // M_s = 0 adds nothing
     zero_acc(acc);
     const Step first = {tb, tb, tb + len, sg, 1, 0};
-    dma_mainloop<false, true, false>(P, o0, n0, first, next, [](const Step&) { return 1.0f; },
+    dma_mainloop<false, false>(P, o0, n0, first, next, [](const Step&) { return 1.0f; },
                                      [](uint16_t*, const Step&) {}, acc);
     const float c = (float)csc[cex[sg]];  // exact: a value of the class dtype
     static_for<BI * BJ>([&](auto q) {
@@ -93,15 +93,13 @@ __device__ __forceinline__ void moments_tile(const int64_t* __restrict__ f, cons
     });
   }
 
-  // Lane holds D[4 (lane >> 4) + e][lane & 15] of each 16 x 16 block.
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wave = threadIdx.x >> 6;
   const int wm = WM * (wave & 1), wn = WN * (wave >> 1);
   static_for<BI * BJ>([&](auto q) {
     constexpr int i = decltype(q)::value / BJ, j = decltype(q)::value % BJ;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int64_t o = o0 + wm + 16 * i + 4 * (lane >> 4) + e;
-      const int64_t n = n0 + wn + 16 * j + (lane & 15);
+      const int64_t o = o0 + wm + acc_row(i), n = n0 + wn + acc_col(j) + e;
       if (o < P.d_out && n < P.d_in) {
         moment_store(out, o * P.d_in + n, odt, s1[i][j][e], normalize_by);
         if (out2 != nullptr) moment_store(out2, o * P.d_in + n, odt, s2[i][j][e], normalize_by);

@@ -16,6 +16,7 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 // moving the read above those writes.
 typedef u32x4_t u32x4_alias_t __attribute__((may_alias));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+typedef u32x2_t u32x2_alias_t __attribute__((may_alias));
 typedef short v4i16_t __attribute__((ext_vector_type(4)));
 
 #ifndef ODP_LIN_OCC
@@ -123,22 +124,21 @@ __device__ __forceinline__ bf16x8_t outer_frag(const uint16_t* tile, int pitch, 
 
 typedef f32x4_t OuterAcc[BI][BJ];
 
-__device__ __forceinline__ void outer_compute(const uint16_t* ta, const uint16_t* tb, OuterAcc& acc) {
-  const int wave = threadIdx.x >> 6;
-  const int wm = WM * (wave & 1), wn = WN * (wave >> 1);
-  // Operand reads run two A fragments ahead of the MFMAs that consume them.
-  bf16x8_t b[BJ], a[3];
-#pragma unroll
-  for (int j = 0; j < BJ; ++j) b[j] = outer_frag(tb, ON, wn + 16 * j);
-  a[0] = outer_frag(ta, OM, wm);
-  a[1] = outer_frag(ta, OM, wm + 16);
-#pragma unroll
-  for (int i = 0; i < BI; ++i) {
-    if (i + 2 < BI) a[(i + 2) % 3] = outer_frag(ta, OM, wm + 16 * (i + 2));
-#pragma unroll
-    for (int j = 0; j < BJ; ++j)
-      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i % 3], b[j], acc[i][j], 0, 0, 0);
-  }
+// Where a lane's accumulator entries lie in the wave's WM x WN block: the
+// MFMAs take X as their first operand, so entry e of block (i, j) is row
+// 16 i + (lane & 15) (an output, column of G) and column 16 j + 4 (lane >>
+// 4) + e (an input, column of X): 4 consecutive elements of a row of M.
+__device__ __forceinline__ int acc_row(int i) { return 16 * i + (int)(threadIdx.x & 15); }
+__device__ __forceinline__ int acc_col(int j) { return 16 * j + 4 * (int)((threadIdx.x & 63) >> 4); }
+
+// The operands a step starts with, read during the step before it.
+struct OuterHead {
+  bf16x8_t b[BJ], a[2];
+};
+
+__device__ __forceinline__ uint32_t uniform32(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+  return ((uint64_t)uniform32((uint32_t)(v >> 32)) << 32) | uniform32((uint32_t)v);
 }
 
 // One pipeline step: rows [t0, t0 + OK) clipped to its segment [tb, te).
@@ -177,8 +177,8 @@ __device__ __forceinline__ u32x4_t scale_bf16x8(u32x4_t v, float c) {
 // Outer-product main loop, buffer loads straight into LDS.  The step's G and
 // X tiles (token-major rows, the XOR swizzle above) are fetched by
 // buffer_load ... lds into a ring of RING LDS stages, RING - 1 steps ahead of
-// the compute, with no staging registers; each step waits for its own loads
-// with an explicit vmcnt and an LDS-only barrier.  The buffer resources
+// the compute, with no staging registers; each step waits for the next
+// step's loads with an explicit vmcnt and an LDS-only barrier.  The buffer resources
 // cover only the rows of the step's segment, so rows outside it (and
 // columns past the matrix, sent past the end) arrive as zeros.  A step never
 // crosses a segment, so the clip factor is one scalar per step; it scales
@@ -193,47 +193,71 @@ constexpr int RPW = OK / NW;                      // tile rows each wave loads p
 #define ODP_LIN_RING 4  // LDS stages of the outer-form ring (RING - 1 steps in flight)
 #endif
 constexpr int RING = ODP_LIN_RING;
-static_assert((RING == 3 || RING == 4) && (RING - 2) * (A_DMA + B_DMA) < 64, "ring depth");
+constexpr int UNROLL = RING % 2 ? 2 * RING : RING;  // steps per loop: stages and operand sets come out even
+static_assert((RING == 4 || RING == 5) && (RING - 2) * (A_DMA + B_DMA) < 64, "ring depth");
 constexpr int DMA_PER_STEP = A_DMA + B_DMA;
 constexpr int B_LPR = ON / 8, B_RPI = 64 / B_LPR;  // X tile: lanes per row, rows per load
 static_assert(OM == 256 && (ON == 128 || ON == 256), "G tile rows take 32 lanes; X tile rows 16 or 32");
 static_assert((NW == 4 || NW == 8) && A_DMA * 2 == RPW && B_DMA * B_RPI == RPW && WN % 16 == 0,
               "each wave loads whole rows of both tiles");
-static_assert(DMA_PER_STEP < 16, "the step wait encodes vmcnt in 4 bits");
+static_assert(DMA_PER_STEP <= BI && BJ < BI, "a step's loads and the next step's operands go out one per block row");
 
-// Column-major over the wave's blocks: X fragment j + 1 is scaled (VALU)
-// while the MFMAs of fragment j run, instead of all scaling up front.
-__device__ __forceinline__ void outer_compute_scaled(const uint16_t* ta, const uint16_t* tb, float c,
-                                                     OuterAcc& acc) {
-  const int wave = threadIdx.x >> 6;
-  const int wm = WM * (wave & 1), wn = WN * (wave >> 1);
-  bf16x8_t a[BI], b[BJ];
-#pragma unroll
-  for (int j = 0; j < BJ; ++j) b[j] = outer_frag(tb, ON, wn + 16 * j);
-#pragma unroll
-  for (int i = 0; i < BI; ++i) a[i] = outer_frag(ta, OM, wm + 16 * i);
-#pragma unroll
-  for (int j = 0; j < BJ; ++j) {
-    const bf16x8_t bs = __builtin_bit_cast(bf16x8_t, scale_bf16x8(__builtin_bit_cast(u32x4_t, b[j]), c));
-#pragma unroll
-    for (int i = 0; i < BI; ++i)
-      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], bs, acc[i][j], 0, 0, 0);
-  }
+// c times an X fragment, rounded to bf16.
+__device__ __forceinline__ bf16x8_t scale_frag(bf16x8_t v, float c) {
+  return __builtin_bit_cast(bf16x8_t, scale_bf16x8(__builtin_bit_cast(u32x4_t, v), c));
 }
 
-// One ring step: loads into stage `nxt`, then the MFMAs from stage `cur`.
-// Both pointers are restrict parameters of one inlined call, which gives
-// the compiler the alias scopes that keep the reads of `cur` from waiting
-// for the loads into `nxt` (without them every LDS read waits for all
-// loads into LDS in flight).
-template <bool SCALE, typename Issue>
+__device__ __forceinline__ void read_head(const uint16_t* st, OuterHead& H) {
+  const int wave = threadIdx.x >> 6;
+  const int wm = WM * (wave & 1), wn = WN * (wave >> 1);
+#pragma unroll
+  for (int j = 0; j < BJ; ++j) H.b[j] = outer_frag(st + A_TILE, ON, wn + 16 * j);
+  H.a[0] = outer_frag(st, OM, wm);
+  H.a[1] = outer_frag(st, OM, wm + 16);
+}
+
+// One ring step: its MFMAs from stage `cur` and the operands in `H`, the
+// loads of a later step into stage `nxt` (issued one by one between the
+// first MFMAs), and the first operands of the next step from stage `ahead`
+// into `N` beside the last MFMAs, so that after the next barrier the MFMAs
+// start at once instead of all eight waves first waiting for their operand
+// reads together (Llama-3-8B-shaped layer, 8 x 4096 tokens: outer norms 1195
+// -> 1270 TFLOP/s with the store and 1279 -> 1350 without, clipped sum 1170
+// -> 1238, moments + 5 %; a fifth stage, one more step of loads in flight,
+// measured + 4 % without the store, nothing with it, and spills in the sum).  The stages are restrict parameters of one inlined call,
+// which gives the compiler the alias scopes that keep the reads from waiting
+// for the loads into `nxt`.  SCALE: X's fragments times `c` (rounded to
+// bf16) before use.  `tick` (the scalar bookkeeping of the step after) runs
+// between the MFMAs, not between the steps, where nothing would cover it.
+template <bool SCALE, typename Issue, typename Tick>
 __device__ __forceinline__ void ring_step(uint16_t* __restrict__ nxt, const uint16_t* __restrict__ cur,
-                                          Issue issue, float c, OuterAcc& acc) {
-  issue(nxt);
-  if (SCALE)
-    outer_compute_scaled(cur, cur + A_TILE, c, acc);
-  else
-    outer_compute(cur, cur + A_TILE, acc);
+                                          const uint16_t* __restrict__ ahead, Issue issue, Tick tick, float c,
+                                          OuterHead& H, OuterHead& N, OuterAcc& acc) {
+  const int wave = threadIdx.x >> 6;
+  const int wm = WM * (wave & 1), wn = WN * (wave >> 1);
+  bf16x8_t a[3];
+  a[0] = H.a[0];
+  a[1] = H.a[1];
+  if (SCALE) {
+#pragma unroll
+    for (int j = 0; j < BJ; ++j) H.b[j] = scale_frag(H.b[j], c);
+  }
+#pragma unroll
+  for (int i = 0; i < BI; ++i) {
+    if (i + 2 < BI) a[(i + 2) % 3] = outer_frag(cur, OM, wm + 16 * (i + 2));
+    if (i < DMA_PER_STEP) issue(nxt, i);
+    if (i >= BI - 1 - BJ && i < BI - 1)
+      N.b[i - (BI - 1 - BJ)] = outer_frag(ahead + A_TILE, ON, wn + 16 * (i - (BI - 1 - BJ)));
+    if (i >= BI - 2) N.a[i - (BI - 2)] = outer_frag(ahead, OM, wm + 16 * (i - (BI - 2)));
+#pragma unroll
+    for (int j = 0; j < BJ; ++j)
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(H.b[j], a[i % 3], acc[i][j], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (i == DMA_PER_STEP - 1) {
+      tick();
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
 }
 
 // The ring: one array per stage, so that reads of one stage are not made to
@@ -242,102 +266,127 @@ __device__ __forceinline__ void ring_step(uint16_t* __restrict__ nxt, const uint
 __shared__ __attribute__((aligned(16))) uint16_t lin_ring0[OUTER_STAGE];
 __shared__ __attribute__((aligned(16))) uint16_t lin_ring1[OUTER_STAGE];
 __shared__ __attribute__((aligned(16))) uint16_t lin_ring2[OUTER_STAGE];
-__shared__ __attribute__((aligned(16))) uint16_t lin_ring3[RING > 3 ? OUTER_STAGE : 8];
+__shared__ __attribute__((aligned(16))) uint16_t lin_ring3[OUTER_STAGE];
+__shared__ __attribute__((aligned(16))) uint16_t lin_ring4[RING > 4 ? OUTER_STAGE : 64];
 __device__ __forceinline__ uint16_t* lin_stage(int k) {
-  return k == 0 ? lin_ring0 : k == 1 ? lin_ring1 : k == 2 ? lin_ring2 : lin_ring3;
+  return k == 0 ? lin_ring0 : k == 1 ? lin_ring1 : k == 2 ? lin_ring2 : k == 3 ? lin_ring3 : lin_ring4;
 }
 
-// DEEP: the step's reads carry alias scopes (ring_step), so they do not
-// wait for the next stage's loads and RING - 1 steps stay in flight.
-// Without it the compiler makes the reads wait for all but the newest
-// loads, one step fewer (every kernel here measured faster with DEEP; the
-// clipped sum by 2 % on C4).
-// FIX: a step whose `fix` is set calls fixup(stage, step) once its loads
-// have landed, then waits for every wave before the MFMAs (segments with
-// non-finite columns only).
-template <bool SCALE, bool DEEP, bool FIX, typename Next, typename Scale, typename Fixup>
+// FIX: a step whose `fix` is set has its stage changed by fixup(stage, step)
+// once its loads have landed, before anything reads it.
+template <bool SCALE, bool FIX, typename Next, typename Scale, typename Fixup>
 __device__ __forceinline__ void dma_mainloop(const LinProblem& P, int64_t o0, int64_t n0, Step first,
                                              Next next, Scale scale, Fixup fixup, OuterAcc& acc) {
-  auto stage = [&](int k) -> uint16_t* { return lin_stage(k); };
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // Per lane: tile row and column of each of its loads (row within the
-  // step, column within the tile after undoing the swizzle).
-  int arow[A_DMA], acol[A_DMA], brow[B_DMA], bcol[B_DMA];
+  // The problem and the steps are the same for every lane; where the compiler
+  // cannot tell (vector loads), it is told.
+  const uint64_t G = uniform64((uint64_t)P.G), X = uniform64((uint64_t)P.X);
+  const uint32_t ldg = uniform32((uint32_t)P.ldg), ldx = uniform32((uint32_t)P.ldx);
+  first = Step{(int32_t)uniform32(first.t0),  (int32_t)uniform32(first.tb),   (int32_t)uniform32(first.te),
+               (int32_t)uniform32(first.seg), (int32_t)uniform32(first.live), (int32_t)uniform32(first.fix)};
+  // Per lane: byte offset of each of its loads from the step's first row
+  // (row within the step, column within the tile after undoing the swizzle;
+  // columns past the matrix go past the end of every buffer).  The step only
+  // moves the buffers' bases, on the scalar unit.
+  uint32_t aoff[A_DMA], boff[B_DMA];
 #pragma unroll
   for (int i = 0; i < A_DMA; ++i) {
-    arow[i] = RPW * wave + 2 * i + (lane >> 5);
-    acol[i] = 8 * ((lane & 31) ^ (swz(arow[i]) >> 1));
+    const int r = RPW * wave + 2 * i + (lane >> 5);
+    const int32_t col = (int32_t)o0 + 8 * ((lane & 31) ^ (swz(r) >> 1));
+    aoff[i] = col < (int32_t)P.d_out ? ((uint32_t)r * ldg + (uint32_t)col) * 2u : LIN_OOB;
   }
 #pragma unroll
   for (int i = 0; i < B_DMA; ++i) {
-    brow[i] = RPW * wave + B_RPI * i + (lane / B_LPR);
-    bcol[i] = 8 * ((lane % B_LPR) ^ (swz(brow[i]) >> 1));
+    const int r = RPW * wave + B_RPI * i + (lane / B_LPR);
+    const int32_t col = (int32_t)n0 + 8 * ((lane % B_LPR) ^ (swz(r) >> 1));
+    boff[i] = col < (int32_t)P.d_in ? ((uint32_t)r * ldx + (uint32_t)col) * 2u : LIN_OOB;
   }
-  const int32_t dout = (int32_t)P.d_out, din = (int32_t)P.d_in;
-  const uint32_t ldg = (uint32_t)P.ldg, ldx = (uint32_t)P.ldx;
 
-  auto issue = [&](uint16_t* st, const Step& x) {
-    const uint32_t rows = x.live ? (uint32_t)(x.te - x.tb) : 0u;
-    const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(P.G + x.tb * P.ldg), (short)0, (int)(rows * ldg * 2u), LIN_BUF_DWORD3);
-    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(P.X + x.tb * P.ldx), (short)0, (int)(rows * ldx * 2u), LIN_BUF_DWORD3);
-    const uint32_t r0 = (uint32_t)(x.t0 - x.tb);
-#pragma unroll
-    for (int i = 0; i < A_DMA; ++i) {
-      const int32_t col = (int32_t)o0 + acol[i];
-      const uint32_t off = col < dout ? ((r0 + arow[i]) * ldg + (uint32_t)col) * 2u : LIN_OOB;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(gr, (ODP_LDS void*)(st + (RPW * wave + 2 * i) * OM), 16, off, 0,
-                                               0, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < B_DMA; ++i) {
-      const int32_t col = (int32_t)n0 + bcol[i];
-      const uint32_t off = col < din ? ((r0 + brow[i]) * ldx + (uint32_t)col) * 2u : LIN_OOB;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (ODP_LDS void*)(st + A_TILE + (RPW * wave + B_RPI * i) * ON),
-                                               16, off, 0, 0, 0);
+  // Where the loads of a step start: its first row of G and of X, and the
+  // bytes from there to the segment's end (rows past it arrive as zeros; a
+  // step past the last one has none).
+  struct LoadAt {
+    uint64_t g, x;
+    uint32_t gbytes, xbytes;
+  };
+  auto load_at = [&](const Step& x) __attribute__((always_inline)) {
+    const uint32_t rows = x.live ? (uint32_t)(x.te - x.t0) : 0u;
+    return LoadAt{G + (uint64_t)x.t0 * ldg * 2u, X + (uint64_t)x.t0 * ldx * 2u, rows * ldg * 2u, rows * ldx * 2u};
+  };
+  // Load i of a step (i < A_DMA: rows of G, then X).
+  auto issue = [&](uint16_t* st, const LoadAt& at, int i) __attribute__((always_inline)) {
+    if (i < A_DMA) {
+      const __amdgpu_buffer_rsrc_t gr =
+          __builtin_amdgcn_make_buffer_rsrc((void*)at.g, (short)0, (int)at.gbytes, LIN_BUF_DWORD3);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(gr, (ODP_LDS void*)(st + (RPW * wave + 2 * i) * OM), 16, aoff[i], 0, 0,
+                                               0);
+    } else {
+      const int k = i - A_DMA;
+      const __amdgpu_buffer_rsrc_t xr =
+          __builtin_amdgcn_make_buffer_rsrc((void*)at.x, (short)0, (int)at.xbytes, LIN_BUF_DWORD3);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (ODP_LDS void*)(st + A_TILE + (RPW * wave + B_RPI * k) * ON), 16,
+                                               boff[k], 0, 0, 0);
     }
   };
 
-  // Prologue: steps 0 .. RING - 2 in flight.  Steps past the last one
-  // still issue (zero rows, so out of range) to keep the wait counts
-  // constant.
+  // Prologue: steps 0 .. RING - 2 in flight, then the operands step 0 starts
+  // with.  Steps past the last one still issue (zero rows, so out of range)
+  // to keep the wait counts constant.
   Step cur = first;
   Step ld = first;
-  float cs[RING];
+  float c = 1.0f;  // of the step `cur`
 #pragma unroll
   for (int q = 0; q < RING - 1; ++q) {
-    issue(stage(q), ld);
-    cs[q] = SCALE && ld.live ? scale(ld) : 1.0f;
+#pragma unroll
+    for (int i = 0; i < DMA_PER_STEP; ++i) issue(lin_stage(q), load_at(ld), i);
     ld = next(ld);
   }
+  LoadAt at = load_at(ld);
+  Step nx = next(cur);
+  // Opaque from here on: left as the constants they start with, the
+  // accumulators of a loop with an exit at every step were kept twice.
+#pragma unroll
+  for (int i = 0; i < BI; ++i)
+#pragma unroll
+    for (int j = 0; j < BJ; ++j) __asm__ volatile("" : "+v"(acc[i][j]));
+  OuterHead H[2];
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm((RING - 2) * DMA_PER_STEP));
+  __asm__ volatile("s_barrier" ::: "memory");
+  if (FIX && __builtin_expect(cur.fix, 0)) {
+    fixup(lin_stage(0), cur);
+    __syncthreads();
+  }
+  read_head(lin_stage(0), H[0]);
+  if (SCALE && cur.live) c = scale(cur);
   while (cur.live) {
 #pragma unroll
-    for (int k = 0; k < RING; ++k) {
+    for (int k = 0; k < UNROLL; ++k) {
       if (!cur.live) break;
-      // This step's loads have landed; the later RING - 2 steps' may fly.
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm((RING - 2) * DMA_PER_STEP));
+      // The next step's loads have landed (this wave's; the barrier says so
+      // for the others); the later RING - 3 steps' may fly.
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm((RING - 3) * DMA_PER_STEP));
       __asm__ volatile("s_barrier" ::: "memory");
-      if (FIX && cur.fix) {
-        fixup(stage(k), cur);
+      if (FIX && __builtin_expect(nx.fix, 0)) {
+        fixup(lin_stage((k + 1) % RING), nx);
         __syncthreads();
       }
       // Loads of step ld go into the stage computed at the previous step.
-      const Step x = ld;
-      const int kn = (k + RING - 1) % RING;
-      if (DEEP) {
-        ring_step<SCALE>(stage(kn), stage(k), [&](uint16_t* st) { issue(st, x); }, cs[k], acc);
-      } else {
-        issue(stage(kn), x);
-        if (SCALE)
-          outer_compute_scaled(stage(k), stage(k) + A_TILE, cs[k], acc);
-        else
-          outer_compute(stage(k), stage(k) + A_TILE, acc);
-      }
-      cs[kn] = SCALE && ld.live ? scale(ld) : 1.0f;
-      ld = next(ld);
-      cur = next(cur);
+      ring_step<SCALE>(lin_stage((k + RING - 1) % RING), lin_stage(k % RING), lin_stage((k + 1) % RING),
+                       [&](uint16_t* st, int i) __attribute__((always_inline)) { issue(st, at, i); },
+                       [&]() __attribute__((always_inline)) {
+                         ld = next(ld);
+                         at = load_at(ld);
+                         cur = nx;
+                         nx = next(nx);
+                         // Computed here, not where they are used: worth
+                         // 4 % of the clipped sum, whose steps cross
+                         // segments (without FIX, a step is an addition
+                         // and pinning it measured 1 % slower).
+                         if (FIX) __asm__ volatile("" : "+s"(at.g), "+s"(at.x), "+s"(at.gbytes), "+s"(at.xbytes));
+                       },
+                       c, H[k & 1], H[(k + 1) & 1], acc);
+      if (SCALE && cur.live) c = scale(cur);
     }
   }
   __builtin_amdgcn_s_waitcnt(0);  // no load into LDS may outlive the workgroup
