@@ -304,6 +304,7 @@ __device__ __forceinline__ void ss_put(void* dst, int64_t o, int odt, bool vec, 
 //         one contiguous run.
 template <int PDT>
 __host__ __device__ constexpr int ss_sg() { return PDT == ODP_DTYPE_F32 ? 8 : 4; }  // 8 KB a wave and group
+constexpr int SS_TILE = SS_THREADS * 8 + SS_THREADS / 4;  // words
 // A transposed tile's element in LDS: one word of skew every 32, so that the
 // column writes (strides of V * rank words) spread over the banks and aligned
 // runs of 8 stay contiguous.
@@ -317,24 +318,16 @@ __device__ __forceinline__ void scale_sum_fast(const void* pe, int64_t M, int ra
   constexpr int V = VEC ? ss_vec<PDT>() : 1, ES = PDT == ODP_DTYPE_F32 ? 4 : 2;
   const int tid = threadIdx.x;
   const int64_t E = M * rank;
-  // Transposed: columns per tile (a multiple of V), pieces per row.
-  const int cols = transpose ? SS_THREADS * V / rank / V * V : 0, ppr = transpose ? cols / V : 1;
+  // Transposed: pieces per thread, columns per tile (a multiple of V; a run of
+  // 128 bytes of a row up to rank 64 in float32, 64 bytes in 16 bits), pieces
+  // per row.
+  constexpr int SUB = PDT == ODP_DTYPE_F32 ? 2 : 1;
+  const int cols = transpose ? SS_THREADS * V * SUB / rank / V * V : 0, ppr = transpose ? cols / V : 1;
   const int64_t ntile = transpose ? (M + cols - 1) / cols : (E + SS_THREADS * V - 1) / (SS_THREADS * V);
   const ODP_CONST int32_t* ex = (const ODP_CONST int32_t*)(sex + seg_first);
   const ODP_CONST double* csc = (const ODP_CONST double*)sc;
-  for (int64_t t = b; t < ntile; t += nblk) {
-    // Element of segment 0 this thread starts at, and how many it has.
-    int64_t e0;
-    bool on;
-    const int k = transpose ? tid / ppr : 0;
-    if (transpose) {
-      const int64_t m = t * cols + (int64_t)(tid % ppr) * V;
-      e0 = (int64_t)k * M + m;
-      on = k < rank && m < M;
-    } else {
-      e0 = t * (SS_THREADS * V) + tid * V;
-      on = e0 < E;
-    }
+  // The finished sums of the piece at element e0 of segment 0, if `on`.
+  auto piece = [&](int64_t e0, bool on, float (&x)[V], float (&x2)[V]) __attribute__((always_inline)) {
     float acc[V], acc2[V];
 #pragma unroll
     for (int i = 0; i < V; ++i) acc[i] = acc2[i] = 0.f;
@@ -375,48 +368,63 @@ __device__ __forceinline__ void scale_sum_fast(const void* pe, int64_t M, int ra
       for (; s + SG <= n_seg; s += SG) group(s, SG);
       if (s < n_seg) group(s, n_seg - s);
     }
-    float x[V], x2[V];
 #pragma unroll
     for (int i = 0; i < V; ++i) {
       x[i] = ss_finish(acc[i], normalize_by, odt);
       if (SECOND) x2[i] = ss_finish(acc2[i], normalize_by, odt);
     }
+  };
+  for (int64_t t = b; t < ntile; t += nblk) {
+    float x[V], x2[V];
+    if constexpr (VEC) if (transpose) {
+      // Tile as [column][rank]: the run out[t * cols * rank ...).
+      const int64_t m0 = t * cols;
+#pragma unroll 1
+      for (int h = 0; h < SUB; ++h) {
+        const int idx = tid + h * SS_THREADS, k = idx / ppr, c0 = (idx - k * ppr) * V;
+        const bool on = k < rank && m0 + c0 < M;
+        piece((int64_t)k * M + m0 + c0, on, x, x2);
+        if (h == 0) __syncthreads();  // the previous tile has been stored
+        if (on) {
+#pragma unroll
+          for (int i = 0; i < V; ++i) {
+            tile[ss_at((c0 + i) * rank + k)] = x[i];
+            if (SECOND) tile[SS_TILE + ss_at((c0 + i) * rank + k)] = x2[i];
+          }
+        }
+      }
+      __syncthreads();
+      const int run = (int)((M - m0 < cols ? M - m0 : cols) * rank);
+      const int oes = odp_dtype_size(odt);
+#pragma unroll 1
+      for (int h = 0; h < (SECOND ? 2 : 1); ++h) {
+        void* dst = h ? out2 : out;
+        const float* src = tile + h * SS_TILE;
+        for (int i = tid * V; i < run; i += SS_THREADS * V) {
+          const int64_t o = m0 * rank + i;
+          if (i + V <= run) {
+#pragma unroll
+            for (int q = 0; q < V; ++q) x[q] = src[ss_at(i) + q];
+            ss_put<V>(dst, o, odt, (((uintptr_t)dst + o * oes) & (V * oes - 1) & 15) == 0, x);
+          } else {
+            for (int q = i; q < run; ++q) odp_store_from_float(dst, m0 * rank + q, odt, src[ss_at(q)]);
+          }
+        }
+      }
+      continue;
+    }
+    const int64_t e0 = t * (SS_THREADS * V) + tid * V;
+    const bool on = e0 < E;
+    piece(e0, on, x, x2);
     if constexpr (!VEC) {
       if (!on) continue;
       odp_store_from_float(out, e0, odt, x[0]);
       if (SECOND) odp_store_from_float(out2, e0, odt, x2[0]);
-    } else if (!transpose) {
+    } else {
       const int oes = odp_dtype_size(odt);
       if (on) {
         ss_put<V>(out, e0, odt, (((uintptr_t)out + e0 * oes) & (V * oes - 1) & 15) == 0, x);
         if (SECOND) ss_put<V>(out2, e0, odt, (((uintptr_t)out2 + e0 * oes) & (V * oes - 1) & 15) == 0, x2);
-      }
-    } else {
-      // Tile as [column][rank]: the run out[t * cols * rank ...).
-      const int64_t m0 = t * cols;
-      const int run = (int)((M - m0 < cols ? M - m0 : cols) * rank);
-#pragma unroll 1
-      for (int h = 0; h < (SECOND ? 2 : 1); ++h) {
-        __syncthreads();
-        if (on) {
-          const int c0 = (tid % ppr) * V;
-#pragma unroll
-          for (int i = 0; i < V; ++i) tile[ss_at((c0 + i) * rank + k)] = SECOND && h ? x2[i] : x[i];
-        }
-        __syncthreads();
-        void* dst = h ? out2 : out;
-        const int oes = odp_dtype_size(odt);
-        for (int i = tid * V; i < run; i += SS_THREADS * V) {
-          const int64_t o = m0 * rank + i;
-          if (i + V <= run) {
-            float y[V];
-#pragma unroll
-            for (int q = 0; q < V; ++q) y[q] = tile[ss_at(i) + q];
-            ss_put<V>(dst, o, odt, (((uintptr_t)dst + o * oes) & (V * oes - 1) & 15) == 0, y);
-          } else {
-            for (int q = i; q < run; ++q) odp_store_from_float(dst, m0 * rank + q, odt, tile[ss_at(q)]);
-          }
-        }
       }
     }
   }
@@ -426,7 +434,7 @@ __global__ __launch_bounds__(SS_THREADS) void k_scale_sum(
     const int64_t* __restrict__ probs, const int32_t* __restrict__ ws, int n_prob,
     const int32_t* __restrict__ sex, const double* __restrict__ scales, int n_ex, int n_groups,
     float normalize_by) {
-  __shared__ float tile[SS_THREADS * 8 + SS_THREADS / 4];
+  __shared__ float tile[2 * SS_TILE];  // sums and second moments of a transposed tile
   const int bid = blockIdx.x;
   const int p = odp_find_problem(ws, n_prob, bid);
   const int64_t* f = probs + (int64_t)p * ODP_SS_FIELDS;

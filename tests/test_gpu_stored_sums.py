@@ -142,3 +142,50 @@ def test_groups_side_by_side(groups):
     assert torch.allclose(res.norms.double(), want.sum(0).sqrt(), rtol=1e-6)
     thr = torch.tensor(C, device=DEV).view(-1, 1)
     assert torch.equal(res.clipped.bool(), res.group_norms > thr.float())
+
+
+@pytest.mark.parametrize("r,frozen", [(8, False), (16, True), (24, False), (64, False)])
+def test_f32_factor_rows(r, frozen):
+    """float32 per-example factor rows (odp_seg_factor): ranks of one to four 16-row blocks, two sites on one
+    activation (one with a frozen A: rows without a leaf), widths of less than a wave's 64 columns, of a
+    workgroup's 256 and past it, segments of less than a step, of several pipelines and unaligned, rows outside
+    the segments NaN.  Each entry is a float32 sum of L products: |error| <= (L + 2) 2^-24 sum |terms|."""
+    print(f"stored sums: fp32 factor rows rank {r} frozen={frozen}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(r)
+    starts, lengths, n_rows = [0, 5, 5, 22, 150], [5, 0, 17, 127, 1], 160
+    seg = Segments(starts, lengths, list(range(5)), 5, n_rows)
+    d_in, outs = 260, (60, 264)
+
+    def rnd(*s):
+        return torch.randn(*s, device=DEV, generator=g)
+
+    inside = torch.zeros(n_rows, dtype=torch.bool, device=DEV)
+    for s, n in zip(starts, lengths):
+        inside[s : s + n] = True
+    x = rnd(n_rows, d_in)
+    x[~inside] = float("nan")
+    sites, leaves = [], []
+    for i, d_out in enumerate(outs):
+        rr = r if i == 0 or r < 64 else 4
+        gt, A, B = rnd(n_rows, d_out), rnd(d_in, rr), rnd(rr, d_out)
+        gt[~inside] = float("nan")
+        a = None
+        if not (frozen and i == 0):
+            a = len(leaves)
+            leaves.append(LeafOut((d_in, rr), torch.float32))
+        leaves.append(LeafOut((rr, d_out), torch.float32))
+        sites.append(LoraSite(x, gt, A, B, 0.5, a_leaf=a, b_leaf=len(leaves) - 1, v=x @ A, u=gt @ B.t()))
+    plan = GhostPlan(segments=seg, leaves=leaves, clip=_clip(leaves, torch.float32, [1e30]), lora_sites=sites,
+                     device=DEV)
+    plan.run()
+    torch.cuda.synchronize()
+    pes = plan.pe_views()
+    for s in sites:
+        for leaf, q, p in ((s.a_leaf, s.u, s.x), (s.b_leaf, s.v, s.g)):
+            if leaf is None:
+                continue
+            got = pes[leaf].view(5, q.shape[1], p.shape[1])
+            for k, (st, n) in enumerate(zip(starts, lengths)):
+                a, b = q[st : st + n].double().t(), p[st : st + n].double()
+                bound = (n + 2) * 2.0**-24 * 0.5 * (a.abs() @ b.abs())
+                assert ((got[k].double() - 0.5 * (a @ b)).abs() <= bound).all(), (leaf, k)
