@@ -178,7 +178,8 @@ int odp_project(odp_stream_t stream, int dtype, const int64_t* problems,
  * waves to part[seg_example[s] * part_stride + slot_base +
  * ODP_FT_WAVE_SLOTS * tile + wave] (a leaf uses ODP_FT_WAVE_SLOTS slots per
  * tile, so no workgroup barrier is needed).  Requirements: M
- * and the P row pitch are multiples of 8 (bf16) or 4 (f32); Q is the output
+ * and the P row pitch are multiples of 8 (bf16) or 4 (f32); f32 rows lie at
+ * least M and less than 128 MiB apart; Q is the output
  * of odp_project (ldq a multiple of 8 and >= n_rows + 32), readable for
  * 16*ceil(r/16) rows; rows k >= r may hold anything (they are discarded). */
 enum {
@@ -260,7 +261,8 @@ int odp_seg_factor_stream(odp_stream_t stream, const int64_t* problems,
  * group w % ODP_FT_GROUPS of its segment w / ODP_FT_GROUPS.  Every leaf
  * starts at a column of Q that is a multiple of 16; a leaf of rank above 16
  * takes the blocks that follow (rank <= 64).  Segments may have any length
- * whose rows span less than 2 GiB of P.  Rows, squares and partial slots as
+ * whose rows span less than 2 GiB of P; the row pitch is at least
+ * ODP_FT_M and less than 16 MiB.  Rows, squares and partial slots as
  * odp_seg_factor's with the same rank blocks, bit for bit.               */
 int odp_seg_factor_stream_tables(odp_stream_t stream, const int64_t* const* problems,
                                  const int32_t* const* block_map, const int32_t* n_prob,

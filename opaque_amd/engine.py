@@ -50,12 +50,23 @@ def _f64_bits(x: float) -> int:
     return struct.unpack("<q", struct.pack("<d", float(x)))[0]
 
 
+# Bytes from one row to the next that 64-token steps address within 32 bits.
+MAX_ROW_PITCH = 1 << 24
+
+
 def _rows(t: torch.Tensor) -> torch.Tensor:
-    """2-D row view [rows, d] with unit column stride and a 16-byte aligned pitch."""
-    t2 = t.reshape(-1, t.shape[-1])
-    align = _ALIGN[t.dtype]
-    if t2.stride(-1) != 1 or t2.stride(0) % align != 0 or t2.data_ptr() % 16 != 0:
-        t2 = t2.contiguous()
+    """2-D row view [rows, d] with unit column stride and a 16-byte aligned
+    pitch of at least d.  The kernels bound a segment's rows by their count
+    times the pitch, so rows that overlap (an expanded activation, the
+    gradient of a sum over tokens) are copied, and rows MAX_ROW_PITCH or more
+    apart too (32-bit offsets that pass a segment's end must not wrap)."""
+    d = t.shape[-1]
+    t2 = t.reshape(-1, d)
+    align, pitch = _ALIGN[t.dtype], t2.stride(0)
+    if t2.stride(-1) != 1 or pitch % align != 0 or t2.data_ptr() % 16 != 0 or pitch < d or \
+            (pitch > d and pitch * t.element_size() >= MAX_ROW_PITCH):
+        # Not contiguous(): it keeps the pitch of a single row.
+        t2 = t2.clone(memory_format=torch.contiguous_format)
     return t2
 
 
@@ -1736,7 +1747,9 @@ class GhostPlan:
         within a segment)."""
         if not self.stream_factors or dt != torch.bfloat16:
             return False
-        return bool(leaves) and all(c % 16 == 0 for c, _ in leaves) and v.max_len * p.stride(0) * 2 < 2**31
+        pitch = p.stride(0) * 2
+        return bool(leaves) and all(c % 16 == 0 for c, _ in leaves) and pitch < MAX_ROW_PITCH \
+            and v.max_len * pitch < 2**31
 
     def _plane_columns(self, ch: list[LoraSite], products: bool) -> list[int]:
         """First column of each site's rank in the chunk's planes.  Planes
