@@ -20,6 +20,7 @@ buffer and uploaded with one asynchronous copy.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 import struct
 import time
@@ -139,11 +140,11 @@ class _SegView:
     def n_rows(self) -> int:
         return self.segs.n_rows
 
-    @property
+    @functools.cached_property
     def valid(self) -> int:
         return int(sum(self.segs.lengths))
 
-    @property
+    @functools.cached_property
     def max_len(self) -> int:
         return max(self.segs.lengths, default=0)
 
@@ -1059,7 +1060,7 @@ class GhostPlan:
         # the others, run the same launch (odp_seg_factor_stream_tables) as
         # different stages.
         limit = int(lib.odp_factor_project_max_len())
-        longest = max((int(t[1].max(initial=0)) for rows in stream_rows.values() for t in rows), default=0)
+        longest = max((t[2].max_len for rows in stream_rows.values() for t in rows), default=0)
         stream_stage = "factor_stream" if longest <= limit else "factor_stream_long"
 
         sq = _Table(N.SQ_FIELDS)
@@ -1768,21 +1769,11 @@ class GhostPlan:
         """A factor problem as rows of the streamed pass: one per segment,
         each leaf's pe rows at the segment's own offset, so that the launch
         can run the most work per workgroup first."""
-        r = int(row[N.FT_R])
-        pe_es = self.pe[torch.bfloat16].element_size()
+        r, valid = int(row[N.FT_R]), v.valid
         ranks = [(row[N.FT_LEAF0 + 3 * li + 1] >> 16) & 0xFFFF for li in range(int(row[N.FT_NLEAF]))]
-        base = np.zeros(N.FT_FIELDS, dtype=np.int64)
-        base[list(row)] = list(row.values())
-        j = np.arange(v.n_seg, dtype=np.int64)
-        rows = np.repeat(base[None], v.n_seg, axis=0)
-        rows[:, N.FT_SEG_FIRST] = v.first + j
-        rows[:, N.FT_NSEG] = 1
-        for li, rk in enumerate(ranks):
-            rows[:, N.FT_LEAF0 + 3 * li] += j * (rk * M * pe_es)
-        ln = np.asarray(v.segs.lengths, dtype=np.int64)
         out.setdefault((r + 15) // 16, []).append(
-            (rows, ln, M, int(((ln * M + planes * r * ln) * es + sum(ranks) * M * es).sum()), int(ln.sum()) * M * es,
-             2 * int(ln.sum()) * M * r))
+            (row, ranks, v, M, (valid * M + planes * r * valid) * es + v.n_seg * sum(ranks) * M * es, valid * M * es,
+             2 * valid * M * r))
 
     def _stream_tables(self, rows: dict[int, list[tuple]]) -> dict[int, _Table]:
         """The streamed rows as one table per rank block count, most work per
@@ -1790,23 +1781,41 @@ class GhostPlan:
         odp_seg_factor_stream_groups()'s size; while the launch would not
         fill the chip STREAM_ROUNDS times, to smaller ones, of at least
         STREAM_MIN_STEPS steps where that still fills it STREAM_MIN_ROUNDS
-        times."""
+        times.  A table's rows are formed at once: problem by problem they
+        are most of a plan's building time."""
+        if not rows:
+            return {}
         lib = N.load()
         slots = STREAM_SLOTS_PER_CU * torch.cuda.get_device_properties(self.device).multi_processor_count \
             if self.device.type == "cuda" else 1
-        tiles = sum((M + 255) // 256 * int((ln > 0).sum()) for lst in rows.values() for _, ln, M, *_ in lst)
+        lengths: dict[int, np.ndarray] = {}
+        for lst in rows.values():
+            for _, _, v, *_ in lst:
+                if id(v) not in lengths:
+                    lengths[id(v)] = np.asarray(v.segs.lengths, dtype=np.int64)
+        live = {k: int((ln > 0).sum()) for k, ln in lengths.items()}
+        tiles = sum((M + 255) // 256 * live[id(v)] for lst in rows.values() for _, _, v, M, *_ in lst)
         per, most = max(1, tiles // (STREAM_ROUNDS * slots)), max(1, tiles // (STREAM_MIN_ROUNDS * slots))
+        pe_es = self.pe[torch.bfloat16].element_size()
+        groups = {M: int(lib.odp_seg_factor_stream_groups(M)) for lst in rows.values() for _, _, _, M, *_ in lst}
         out: dict[int, _Table] = {}
         for nkb in sorted(rows):
-            work = []
-            for arr, ln, M, *_ in rows[nkb]:
-                n = (M + 255) // 256
-                size = np.maximum(per, np.minimum(most, -(-STREAM_MIN_STEPS // np.maximum((ln + 63) // 64, 1))))
-                arr[:, N.FT_GROUPS] = np.maximum(int(lib.odp_seg_factor_stream_groups(M)), -(-n // size))
-                work.append(ln * M / arr[:, N.FT_GROUPS])
-            order = np.argsort(-np.concatenate(work), kind="stable")
-            arr = np.concatenate([t[0] for t in rows[nkb]])[order]
-            out[nkb] = _MappedTable(arr, arr[:, N.FT_GROUPS], *(sum(t[k] for t in rows[nkb]) for k in (3, 5, 4)))
+            lst = rows[nkb]
+            base = np.array([[row.get(f, 0) for f in range(N.FT_FIELDS)] for row, *_ in lst], dtype=np.int64)
+            n_seg = np.array([t[2].n_seg for t in lst])
+            prob = np.repeat(np.arange(len(lst)), n_seg)
+            j = np.arange(len(prob)) - (np.cumsum(n_seg) - n_seg)[prob]
+            ln = np.concatenate([lengths[id(t[2])] for t in lst])
+            arr = base[prob]
+            arr[:, N.FT_SEG_FIRST] = np.array([t[2].first for t in lst])[prob] + j
+            arr[:, N.FT_NSEG] = 1
+            step = np.array([[rk * t[3] * pe_es for rk in (t[1] + [0, 0, 0])[:4]] for t in lst], dtype=np.int64)
+            arr[:, N.FT_LEAF0 : N.FT_LEAF0 + 12 : 3] += j[:, None] * step[prob]
+            M, floor = np.array([[t[3], groups[t[3]]] for t in lst], dtype=np.int64)[prob].T
+            size = np.maximum(per, np.minimum(most, -(-STREAM_MIN_STEPS // np.maximum((ln + 63) // 64, 1))))
+            ng = arr[:, N.FT_GROUPS] = np.maximum(floor, -(-((M + 255) // 256) // size))
+            arr = arr[np.argsort(-(ln * M / ng), kind="stable")]
+            out[nkb] = _MappedTable(arr, arr[:, N.FT_GROUPS], *(sum(t[k] for t in lst) for k in (4, 6, 5)))
         return out
 
     def _a_row(self, x, d_in, qaddr, ubase, col0, r, ldq, seg_first, n_seg, scaling, leaves, pe_off, slot_base):
