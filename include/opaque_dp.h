@@ -178,8 +178,7 @@ int odp_project(odp_stream_t stream, int dtype, const int64_t* problems,
  * waves to part[seg_example[s] * part_stride + slot_base +
  * ODP_FT_WAVE_SLOTS * tile + wave] (a leaf uses ODP_FT_WAVE_SLOTS slots per
  * tile, so no workgroup barrier is needed).  Requirements: M
- * and the P row pitch are multiples of 8 (bf16) or 4 (f32); f32 rows lie at
- * least M and less than 128 MiB apart; Q is the output
+ * and the P row pitch are multiples of 8 (bf16) or 4 (f32); Q is the output
  * of odp_project (ldq a multiple of 8 and >= n_rows + 32), readable for
  * 16*ceil(r/16) rows; rows k >= r may hold anything (they are discarded). */
 enum {

@@ -1163,16 +1163,19 @@ __global__ __launch_bounds__(256, ps_ring(NKB) == 2 ? 2 : 1) void k_project_stre
 constexpr int FF_T = 16;      // tokens per step
 constexpr int FF_DEPTH = 4;   // steps in flight
 
-template <int NKB>
-__global__ __launch_bounds__(256) void k_factor_f32(const int64_t* __restrict__ probs,
-                                                    const int32_t* __restrict__ ws, int n_prob,
-                                                    const int32_t* __restrict__ sstart,
-                                                    const int32_t* __restrict__ slen,
-                                                    const int32_t* __restrict__ sex,
-                                                    double* __restrict__ part, int64_t part_stride) {
-  const int bid = blockIdx.x;
-  const int p = odp_find_problem(ws, n_prob, bid);
-  const int64_t* f = probs + (int64_t)p * ODP_FT_FIELDS;
+// Rows whose offsets within a step pass 31 bits (FAR: a pitch of about 143 MB
+// and more, or below 0) are read by 64-bit addresses; every other pitch, down
+// to rows that overlap, takes the buffer loads.
+__device__ __forceinline__ bool factor_f32_far(int64_t ldp, int64_t M) {
+  constexpr int64_t LIM = (int64_t)1 << 29;  // elements
+  return ldp < 0 || ldp >= LIM || M >= LIM || (FF_T - 1) * ldp + M > LIM;
+}
+
+template <int NKB, bool FAR>
+__device__ __forceinline__ void factor_f32(const int64_t* __restrict__ f, int local,
+                                           const int32_t* __restrict__ sstart, const int32_t* __restrict__ slen,
+                                           const int32_t* __restrict__ sex, double* __restrict__ part,
+                                           int64_t part_stride) {
   const float* P = (const float*)f[ODP_FT_P];
   const int64_t ldp = f[ODP_FT_LDP], M = f[ODP_FT_M];
   const float* Q = (const float*)f[ODP_FT_Q];
@@ -1182,7 +1185,6 @@ __global__ __launch_bounds__(256) void k_factor_f32(const int64_t* __restrict__ 
   const float scale = (float)__longlong_as_double(f[ODP_FT_SCALING]);
 
   const int ntile = (int)((M + FT_M_F32 - 1) / FT_M_F32);
-  const int local = bid - ws[p];
   const int seg = local / ntile, tile = local - seg * ntile;
   const int gs = seg_first + seg;
   const int32_t rs = sstart[gs], t_hi = rs + slen[gs];
@@ -1196,21 +1198,31 @@ __global__ __launch_bounds__(256) void k_factor_f32(const int64_t* __restrict__ 
   struct Stage {
     f32x4_t p[4], q[NKB];
   };
-  // Loads of step s.  P through a buffer over the step's rows of the segment:
-  // rows outside (offsets before it wrap past its end) and columns past M
-  // arrive as zeros; a step past the last one has no rows.
+  // Loads of step s.  P through a buffer at the step's first row of the
+  // segment: rows outside the segment and columns past M are sent past its
+  // end and arrive as zeros.
   const uint32_t ldb = (uint32_t)ldp * 4u;
   const uint32_t mb = m0 < M ? (uint32_t)m0 * 4u : 0x80000000u;
   auto load = [&](int s, Stage& S) {
     const int32_t t0 = t_lo + s * FF_T, lo = t0 > rs ? t0 : rs, hi = t0 + FF_T < t_hi ? t0 + FF_T : t_hi;
-    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(P + (int64_t)(lo < t_hi ? lo : rs) * ldp), (short)0, hi > lo ? (int)((uint32_t)(hi - lo) * ldb) : 0,
-        ODP_BUFFER_DWORD3);
     const int32_t tb = t0 + 4 * g;
+    if constexpr (FAR) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const uint32_t off = mb == 0x80000000u || tb + q < lo ? 0x80000000u : (uint32_t)(tb + q - lo) * ldb + mb;
-      S.p[q] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, FP_G_NT));
+      for (int q = 0; q < 4; ++q) {
+        S.p[q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if (m0 < M && tb + q >= lo && tb + q < hi)
+          S.p[q] = __builtin_bit_cast(f32x4_t, ld16(P + (int64_t)(tb + q) * ldp + m0));
+      }
+    } else {
+      const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(P + (int64_t)(lo < t_hi ? lo : rs) * ldp), (short)0, (int)0x80000000u, ODP_BUFFER_DWORD3);
+      const uint32_t rows = hi > lo ? (uint32_t)(hi - lo) : 0u;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t row = (uint32_t)(tb + q - lo);
+        const uint32_t off = mb == 0x80000000u || row >= rows ? 0x80000000u : row * ldb + mb;
+        S.p[q] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, FP_G_NT));
+      }
     }
     const int64_t tq = tb < t_hi ? tb : t_lo;
 #pragma unroll
@@ -1304,6 +1316,22 @@ __global__ __launch_bounds__(256) void k_factor_f32(const int64_t* __restrict__ 
       if (lane == 0) odp_gstore(part + (int64_t)ex * part_stride + L.slot[q] + ODP_FT_WAVE_SLOTS * tile + wave, v);
     }
   }
+}
+
+template <int NKB>
+__global__ __launch_bounds__(256) void k_factor_f32(const int64_t* __restrict__ probs,
+                                                    const int32_t* __restrict__ ws, int n_prob,
+                                                    const int32_t* __restrict__ sstart,
+                                                    const int32_t* __restrict__ slen,
+                                                    const int32_t* __restrict__ sex,
+                                                    double* __restrict__ part, int64_t part_stride) {
+  const int p = odp_find_problem(ws, n_prob, blockIdx.x);
+  const int64_t* f = probs + (int64_t)p * ODP_FT_FIELDS;
+  const int local = blockIdx.x - ws[p];
+  if (factor_f32_far(f[ODP_FT_LDP], f[ODP_FT_M]))
+    factor_f32<NKB, true>(f, local, sstart, slen, sex, part, part_stride);
+  else
+    factor_f32<NKB, false>(f, local, sstart, slen, sex, part, part_stride);
 }
 
 }  // namespace

@@ -6,6 +6,7 @@ gradient of a sum over tokens) or overlapping rows would read as zeros past
 that bound, and rows 16 MiB or more apart could wrap a 32-bit offset back into
 it.  Such inputs are copied; every plan over them equals, bit for bit, the
 plan over contiguous copies, and the rows it stores equal the float64 product.
+odp_seg_factor itself takes float32 rows of any pitch.
 """
 
 from __future__ import annotations
@@ -96,3 +97,54 @@ def test_factor_rows_of_any_pitch(kind, rank, dt):
         for got, w in zip(outs[0], want):
             err = (got.double().view(w.shape) - w).norm() / w.norm()
             assert err < eps + 8 * torch.finfo(torch.float32).eps, (side, kind, float(err))
+
+
+# Elements from one row to the next: one row for all, rows that overlap, the row itself, a padded row, and rows
+# on both sides of the pitch whose offsets within a step pass 31 bits (128 MiB and 160 MiB).
+F32_PITCHES = {"expanded": 0, "overlapping": 8, "contiguous": 264, "padded": 272, "128MiB": 1 << 25, "160MiB": 5 << 23}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rank", [3, 20, 64])
+@pytest.mark.parametrize("kind", sorted(F32_PITCHES))
+def test_f32_factor_entry_takes_any_pitch(kind, rank):
+    """odp_seg_factor called directly.  Each entry is a float32 sum of at most 18 products: |error| <= (n + 2)
+    2^-24 sum |terms|."""
+    print(f"row pitch: odp_seg_factor f32, {kind} rank {rank}", flush=True)
+    lib, M, pitch = N.load(), 264, F32_PITCHES[kind]
+    starts, lens = [0, 2], [1, 18]  # one row, and an unaligned segment of two steps
+    rows = sum(lens) + 1
+    if pitch > 1000:
+        starts, lens, rows = [0, 1], [1, 3], 4
+    g = torch.Generator(device="cuda").manual_seed(rank)
+    base = torch.empty(pitch * (rows - 1) + M, device="cuda")
+    P = base.as_strided((rows, M), (pitch, 1))
+    if pitch < M:
+        base.copy_(torch.randn(base.shape, device="cuda", generator=g))
+    else:
+        P.copy_(torch.randn(rows, M, device="cuda", generator=g))
+    nkb, ldq = (rank + 15) // 16, (rows + 32 + 7) // 8 * 8
+    Q = torch.randn(16 * nkb, ldq, device="cuda", generator=g)
+    pe = torch.zeros(2, rank, M, device="cuda")
+    slots = N.FT_WAVE_SLOTS * int(lib.odp_seg_factor_tiles(N.DTYPE_F32, M, rank))
+    part = torch.zeros(2, slots, device="cuda", dtype=torch.float64)
+    row = [0] * N.FT_FIELDS
+    row[N.FT_P], row[N.FT_LDP], row[N.FT_M] = P.data_ptr(), pitch, M
+    row[N.FT_Q], row[N.FT_LDQ], row[N.FT_R] = Q.data_ptr(), ldq, rank
+    row[N.FT_NSEG], row[N.FT_NLEAF] = 2, 1
+    row[N.FT_SCALING] = int(torch.tensor([0.5], dtype=torch.float64).view(torch.int64).item())
+    row[N.FT_LEAF0], row[N.FT_LEAF0 + 1] = pe.data_ptr(), rank << 16
+    blocks = 2 * slots // N.FT_WAVE_SLOTS
+    dev = [torch.tensor(v, device="cuda", dtype=dt) for v, dt in
+           ((row, torch.int64), ([0, blocks], torch.int32), (starts, torch.int32), (lens, torch.int32),
+            ([0, 1], torch.int32))]
+    probs, ws, sst, sln, sex = (t.data_ptr() for t in dev)
+    N.check(lib.odp_seg_factor(torch.cuda.current_stream().cuda_stream, N.DTYPE_F32, probs, ws, 1, blocks, sst, sln,
+                               sex, part.data_ptr(), slots, nkb), kind)
+    torch.cuda.synchronize()
+    for k, (st, n) in enumerate(zip(starts, lens)):
+        a, b = Q[:rank, st : st + n].double(), P[st : st + n].double()
+        bound = (n + 2) * 2.0**-24 * 0.5 * (a.abs() @ b.abs())
+        assert ((pe[k].double() - 0.5 * (a @ b)).abs() <= bound).all(), (kind, k)
+        # float32 squares in fp64: each rounds by at most 2^-24 of itself.
+        assert torch.allclose(part[k].sum(), pe[k].double().square().sum(), rtol=2.0**-23)
