@@ -1236,9 +1236,12 @@ __device__ __forceinline__ void factor_f32(const int64_t* __restrict__ f, int lo
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb) acc[j][kb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
+  // An empty segment reads nothing: its start may lie anywhere.
   Stage S[FF_DEPTH];
+  if (nsteps > 0) {
 #pragma unroll
-  for (int d = 0; d < FF_DEPTH; ++d) load(d, S[d]);
+    for (int d = 0; d < FF_DEPTH; ++d) load(d, S[d]);
+  }
   for (int s = 0; s < nsteps; s += FF_DEPTH) {
 #pragma unroll
     for (int d = 0; d < FF_DEPTH; ++d) {

@@ -112,10 +112,10 @@ def test_f32_factor_entry_takes_any_pitch(kind, rank):
     2^-24 sum |terms|."""
     print(f"row pitch: odp_seg_factor f32, {kind} rank {rank}", flush=True)
     lib, M, pitch = N.load(), 264, F32_PITCHES[kind]
-    starts, lens = [0, 2], [1, 18]  # one row, and an unaligned segment of two steps
-    rows = sum(lens) + 1
+    # One row, an unaligned segment of two steps, and an empty one whose start lies past every row: it reads nothing.
+    starts, lens, rows = [0, 2, 1 << 30], [1, 18, 0], 20
     if pitch > 1000:
-        starts, lens, rows = [0, 1], [1, 3], 4
+        starts, lens, rows = [0, 1, 1 << 30], [1, 3, 0], 4
     g = torch.Generator(device="cuda").manual_seed(rank)
     base = torch.empty(pitch * (rows - 1) + M, device="cuda")
     P = base.as_strided((rows, M), (pitch, 1))
@@ -125,24 +125,27 @@ def test_f32_factor_entry_takes_any_pitch(kind, rank):
         P.copy_(torch.randn(rows, M, device="cuda", generator=g))
     nkb, ldq = (rank + 15) // 16, (rows + 32 + 7) // 8 * 8
     Q = torch.randn(16 * nkb, ldq, device="cuda", generator=g)
-    pe = torch.zeros(2, rank, M, device="cuda")
+    pe = torch.ones(3, rank, M, device="cuda")
     slots = N.FT_WAVE_SLOTS * int(lib.odp_seg_factor_tiles(N.DTYPE_F32, M, rank))
-    part = torch.zeros(2, slots, device="cuda", dtype=torch.float64)
+    part = torch.zeros(3, slots, device="cuda", dtype=torch.float64)
     row = [0] * N.FT_FIELDS
     row[N.FT_P], row[N.FT_LDP], row[N.FT_M] = P.data_ptr(), pitch, M
     row[N.FT_Q], row[N.FT_LDQ], row[N.FT_R] = Q.data_ptr(), ldq, rank
-    row[N.FT_NSEG], row[N.FT_NLEAF] = 2, 1
+    row[N.FT_NSEG], row[N.FT_NLEAF] = 3, 1
     row[N.FT_SCALING] = int(torch.tensor([0.5], dtype=torch.float64).view(torch.int64).item())
     row[N.FT_LEAF0], row[N.FT_LEAF0 + 1] = pe.data_ptr(), rank << 16
-    blocks = 2 * slots // N.FT_WAVE_SLOTS
+    blocks = 3 * slots // N.FT_WAVE_SLOTS
     dev = [torch.tensor(v, device="cuda", dtype=dt) for v, dt in
            ((row, torch.int64), ([0, blocks], torch.int32), (starts, torch.int32), (lens, torch.int32),
-            ([0, 1], torch.int32))]
+            ([0, 1, 2], torch.int32))]
     probs, ws, sst, sln, sex = (t.data_ptr() for t in dev)
     N.check(lib.odp_seg_factor(torch.cuda.current_stream().cuda_stream, N.DTYPE_F32, probs, ws, 1, blocks, sst, sln,
                                sex, part.data_ptr(), slots, nkb), kind)
     torch.cuda.synchronize()
     for k, (st, n) in enumerate(zip(starts, lens)):
+        if n == 0:
+            assert not pe[k].any() and not part[k].any()
+            continue
         a, b = Q[:rank, st : st + n].double(), P[st : st + n].double()
         bound = (n + 2) * 2.0**-24 * 0.5 * (a.abs() @ b.abs())
         assert ((pe[k].double() - 0.5 * (a @ b)).abs() <= bound).all(), (kind, k)
