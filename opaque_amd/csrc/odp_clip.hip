@@ -16,6 +16,7 @@ namespace {
 
 constexpr int CL_THREADS = 1024;  // one workgroup per example
 constexpr int CL_DEPTH = 8;      // loads in flight per thread (a power of two)
+constexpr int CL_LONG = 16 * 64 * CL_DEPTH * 2;  // partials a wave sums in 16 rounds of loads
 constexpr int CL_MAX_GROUPS = 1024;
 static_assert(CL_MAX_GROUPS <= CL_THREADS, "thread g finishes group g");
 constexpr int SS_THREADS = 256;
@@ -41,8 +42,14 @@ __device__ __forceinline__ double finalize_scale(double ratio, double rel, doubl
 // and lane reads, then the group's waves in order), so runs are bitwise
 // reproducible.  Several groups are summed side by side, the 16 waves split
 // evenly among them: one after the other, each by the whole workgroup, they
-// are a chain of load latencies and barriers (14 groups of 584 partials: 19
-// us, 7 us side by side; one group: 6 us either way).
+// are a chain of load latencies and barriers (14 groups of 584 partials: 16
+// us, 5 us side by side; one group: 6 us either way).  A group far longer than
+// the others, left on one or two waves, would be summed by them alone (about
+// 0.3 us a wave for 1024 partials), so it takes the whole workgroup after the
+// rest: past CL_LONG partials a wave (below, a round of all the waves costs
+// what it saves) and four times its waves' even share (one of 40960 among
+// 16: 17 -> 9 us, of 200000: 67 -> 18; 16 of 8192 each stay side by side, 11 us
+// against 23).
 // `status` (optional): a word that k_sqnorm sets when it dropped a write
 // outside the partials; every example then gets a NaN norm, zero scales and
 // clear masks, since the partials are incomplete.
@@ -69,7 +76,7 @@ __global__ __launch_bounds__(CL_THREADS) void k_clip_factors(
   __shared__ double red[CL_THREADS / 64];
   __shared__ double gsq[CL_MAX_GROUPS];
   __shared__ double sguard[16];
-  __shared__ int scls[8];
+  __shared__ int scls[8], slong[CL_THREADS / 64];
   const double* row = part + (int64_t)ex * n_slots;
   // The inputs of the scale arithmetic are read now, so that their load
   // latency overlaps the partials' instead of following the reduction
@@ -79,56 +86,81 @@ __global__ __launch_bounds__(CL_THREADS) void k_clip_factors(
   if (t < 2 * n_cls) sguard[t] = guard[t];
   if (t < n_cls) scls[t] = cls_dtype[t];
 
+  // This wave's part of the sum of slots [lo, hi), taken by nth threads of
+  // which this is the tg-th (the same in every lane).
+  auto sum_slots = [&](int64_t lo, int64_t hi, int tg, int nth) __attribute__((always_inline)) {
+    double a[CL_DEPTH];
+#pragma unroll
+    for (int q = 0; q < CL_DEPTH; ++q) a[q] = 0.0;
+    // Slots are read in 16-byte pairs from the first 16-byte aligned one (by
+    // address, so any 8-byte aligned partials buffer works; a leading and a
+    // trailing odd slot go to the group's first thread), and every load of a
+    // round is issued before the first add (masked past the group's end).
+    int64_t la = lo + (int64_t)((((uintptr_t)(row + lo)) >> 3) & 1u);
+    la = la < hi ? la : hi;
+    const int64_t npair = (hi - la) >> 1;
+    if (tg == 0) {
+      if (lo < la) a[0] += row[lo];
+      if (la + 2 * npair < hi) a[1] += row[hi - 1];
+    }
+    const double2* pr = (const double2*)(row + la);
+    for (int64_t q0 = tg; q0 < npair; q0 += CL_DEPTH * nth) {
+      double2 v[CL_DEPTH];
+#pragma unroll
+      for (int q = 0; q < CL_DEPTH; ++q)
+        v[q] = q0 + q * nth < npair ? pr[q0 + q * nth] : double2{0.0, 0.0};
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < CL_DEPTH; ++q) a[q] = (a[q] + v[q].x) + v[q].y;
+    }
+    // Pairwise over the accumulators, in a fixed order.
+#pragma unroll
+    for (int w = CL_DEPTH / 2; w > 0; w >>= 1)
+#pragma unroll
+      for (int q = 0; q < w; ++q) a[q] = a[2 * q] + a[2 * q + 1];
+    return rows_sum4(row_sum16(a[0]));
+  };
   // Waves per group: 16 for one group, halved until the groups fit side by
   // side (one wave each beyond 8 groups, in rounds of 16 groups).
   constexpr int NWAVE = CL_THREADS / 64;
   int wpg = NWAVE;
   while (wpg > 1 && wpg * n_groups > NWAVE) wpg >>= 1;
-  const int wave = t >> 6, nth = 64 * wpg, tg = t & (nth - 1);
+  // Four waves come close to what the CU can have in flight, so a group on
+  // four or more needs no help.
+  const bool few = wpg < 4;
+  const int64_t all = few ? gstart[n_groups] - gstart[0] : 0;
+  auto is_long = [&](int64_t n) { return few && n > (int64_t)CL_LONG * wpg && 4 * n > wpg * all; };
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), nth = 64 * wpg, tg = t & (nth - 1);
+  if (few && t < NWAVE) slong[t] = 0;
   for (int g0 = 0; g0 < n_groups; g0 += NWAVE / wpg) {
     const int g = g0 + wave / wpg;
-    double a[CL_DEPTH];
-#pragma unroll
-    for (int q = 0; q < CL_DEPTH; ++q) a[q] = 0.0;
-    if (g < n_groups) {
-      // Slots are read in 16-byte pairs from the first 16-byte aligned one
-      // (by address, so any 8-byte aligned partials buffer works; a leading
-      // and a trailing odd slot go to the group's first thread), and every
-      // load of a round is issued before the first add (masked past the
-      // group's end).
-      const int64_t lo = gstart[g], hi = gstart[g + 1];
-      int64_t la = lo + (int64_t)((((uintptr_t)(row + lo)) >> 3) & 1u);
-      la = la < hi ? la : hi;
-      const int64_t npair = (hi - la) >> 1;
-      if (tg == 0) {
-        if (lo < la) a[0] += row[lo];
-        if (la + 2 * npair < hi) a[1] += row[hi - 1];
-      }
-      const double2* pr = (const double2*)(row + la);
-      for (int64_t q0 = tg; q0 < npair; q0 += CL_DEPTH * nth) {
-        double2 v[CL_DEPTH];
-#pragma unroll
-        for (int q = 0; q < CL_DEPTH; ++q)
-          v[q] = q0 + q * nth < npair ? pr[q0 + q * nth] : double2{0.0, 0.0};
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int q = 0; q < CL_DEPTH; ++q) a[q] = (a[q] + v[q].x) + v[q].y;
-      }
-      // Pairwise over the accumulators, in a fixed order.
-#pragma unroll
-      for (int w = CL_DEPTH / 2; w > 0; w >>= 1)
-#pragma unroll
-        for (int q = 0; q < w; ++q) a[q] = a[2 * q] + a[2 * q + 1];
-    }
-    const double ws = rows_sum4(row_sum16(a[0]));
+    const int64_t lo = g < n_groups ? gstart[g] : 0, hi = g < n_groups ? gstart[g + 1] : 0;
+    const bool longer = is_long(hi - lo);
+    const double ws = sum_slots(lo, longer ? lo : hi, tg, nth);
     if ((t & 63) == 0) red[wave] = ws;
     __syncthreads();
     if (g < n_groups && tg == 0) {
       double tot = 0.0;
       for (int w = 0; w < wpg; ++w) tot += red[wave + w];
       gsq[g] = tot;
+      if (longer) slong[wave] = 1;
     }
     __syncthreads();
+  }
+  if (few && __builtin_amdgcn_ballot_w64(slong[t & (NWAVE - 1)] != 0) != 0) {
+    for (int g = 0; g < n_groups; ++g) {
+      const int64_t lo = gstart[g], hi = gstart[g + 1];
+      if (!is_long(hi - lo)) continue;  // the same for every thread
+      const double ws = sum_slots(lo, hi, t, CL_THREADS);
+      if ((t & 63) == 0) red[wave] = ws;
+      __syncthreads();
+      if (t == 0) {
+        double tot = 0.0;
+        for (int w = 0; w < NWAVE; ++w) tot += red[w];
+        gsq[g] = tot;
+      }
+      __syncthreads();
+    }
   }
 
   if (t == 0) {

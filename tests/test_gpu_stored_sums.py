@@ -189,3 +189,49 @@ def test_f32_factor_rows(r, frozen):
                 a, b = q[st : st + n].double().t(), p[st : st + n].double()
                 bound = (n + 2) * 2.0**-24 * 0.5 * (a.abs() @ b.abs())
                 assert ((got[k].double() - 0.5 * (a @ b)).abs() <= bound).all(), (leaf, k)
+
+
+# Partials per group: a group goes to the whole workgroup past 16384 partials a wave and four times its waves'
+# even share (five to eight groups have two waves each, more have one).
+LONG = {
+    "one_of_sixteen": [64] * 7 + [40961] + [63] * 8,
+    "at_the_limit": [1] * 9 + [16384],
+    "past_the_limit": [1] * 9 + [16385],
+    "two_waves": [3, 50001, 0, 7, 1],
+    "three_long": [40000, 1, 2, 40001, 5, 6, 7, 39999, 9, 10],
+    "last_of_forty": [17] * 39 + [100003],
+    "even": [20000] * 10,
+}
+
+
+@pytest.mark.parametrize("name", sorted(LONG))
+def test_one_long_group_among_short_ones(name):
+    """odp_clip_factors called directly on partials of one group layout; fp64 sums in some order: rel 1e-6 of the
+    float32 results, and the same bits from run to run."""
+    print(f"stored sums: clip groups {name}", flush=True)
+    lib, lens, n_ex = N.load(), LONG[name], 3
+    g = torch.Generator(device=DEV).manual_seed(len(lens))
+    part = torch.rand(n_ex, sum(lens), device=DEV, dtype=torch.float64, generator=g)
+    bounds = [sum(lens[:k]) for k in range(len(lens) + 1)]
+    want = torch.stack([part[:, a:b].sum(1) for a, b in zip(bounds, bounds[1:])])
+    thr = want.sqrt().mean(1) + 0.5
+    start = torch.tensor(bounds, device=DEV, dtype=torch.int64)
+    guard, cls = torch.tensor([1.0, 0.0], device=DEV, dtype=torch.float64), torch.zeros(1, device=DEV, dtype=torch.int32)
+    runs = []
+    for _ in range(2):
+        scales = torch.zeros(1, len(lens), n_ex, device=DEV, dtype=torch.float64)
+        norms, gn = torch.zeros(n_ex, device=DEV), torch.zeros(len(lens), n_ex, device=DEV)
+        clipped = torch.zeros(len(lens), n_ex, device=DEV, dtype=torch.uint8)
+        total = torch.zeros(n_ex, device=DEV, dtype=torch.uint8)
+        N.check(lib.odp_clip_factors(torch.cuda.current_stream().cuda_stream, part.data_ptr(), part.shape[1], n_ex,
+                                     start.data_ptr(), len(lens), thr.data_ptr(), 1.0, N.CLIP_FIXED, 0.0, 1,
+                                     guard.data_ptr(), cls.data_ptr(), scales.data_ptr(), norms.data_ptr(),
+                                     gn.data_ptr(), clipped.data_ptr(), total.data_ptr()), name)
+        runs.append((scales, norms, gn, clipped, total))
+    torch.cuda.synchronize()
+    scales, norms, gn, clipped, _ = runs[0]
+    assert torch.allclose(gn.double(), want.sqrt(), rtol=1e-6)
+    assert torch.allclose(norms.double(), want.sum(0).sqrt(), rtol=1e-6)
+    assert torch.allclose(scales[0], (thr.view(-1, 1) / want.sqrt()).clamp(max=1.0), rtol=1e-6)
+    assert torch.equal(clipped.bool(), gn > thr.float().view(-1, 1))
+    assert all(torch.equal(a, b) for a, b in zip(*runs))
