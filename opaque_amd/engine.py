@@ -342,29 +342,29 @@ class GhostResult:
 
 
 class _Pack:
-    """Collects host arrays and uploads them with one pinned async copy."""
+    """Collects host arrays and uploads them with one pinned async copy.
+    ``fixed`` arrays (segment arrays, work starts, launch maps) lie behind the
+    others: refresh() copies only those a rebound plan patches."""
 
     def __init__(self) -> None:
         self._chunks: list[np.ndarray] = []
-        self._offsets: list[int] = []
-        self._size = 0
+        self._fixed: list[bool] = []
 
-    def add(self, arr: np.ndarray) -> int:
-        arr = np.ascontiguousarray(arr)
-        off = (self._size + 255) // 256 * 256
-        self._chunks.append(arr)
-        self._offsets.append(off)
-        self._size = off + arr.nbytes
+    def add(self, arr: np.ndarray, fixed: bool = False) -> int:
+        self._chunks.append(np.ascontiguousarray(arr))
+        self._fixed.append(fixed)
         return len(self._chunks) - 1
 
     def array(self, i: int) -> np.ndarray:
         return self._chunks[i]
 
-    def _pinned(self) -> torch.Tensor:
-        host = torch.empty(max(self._size, 1), dtype=torch.uint8, pin_memory=True)
+    def _pinned(self, size: int) -> torch.Tensor:
+        """The arrays in the first ``size`` bytes of the buffer."""
+        host = torch.empty(max(size, 1), dtype=torch.uint8, pin_memory=True)
         hn = host.numpy()
         for arr, off in zip(self._chunks, self._offsets):
-            hn[off : off + arr.nbytes] = arr.view(np.uint8).reshape(-1)
+            if off + arr.nbytes <= size:
+                hn[off : off + arr.nbytes] = arr.view(np.uint8).reshape(-1)
         return host
 
     def refresh(self) -> None:
@@ -372,10 +372,18 @@ class _Pack:
         copy is ordered on the current stream after earlier launches that read
         the buffer; torch's pinned-memory allocator keeps the source alive
         until the copy is done."""
-        self._dev.copy_(self._pinned(), non_blocking=True)
+        self._dev[: max(self._patched, 1)].copy_(self._pinned(self._patched), non_blocking=True)
 
     def upload(self, device: torch.device) -> list[torch.Tensor]:
-        dev = self._pinned().to(device, non_blocking=True)
+        self._offsets, size = [0] * len(self._chunks), 0
+        for fixed in (False, True):
+            for i, arr in enumerate(self._chunks):
+                if self._fixed[i] == fixed:
+                    self._offsets[i] = (size + 255) // 256 * 256
+                    size = self._offsets[i] + arr.nbytes
+            if not fixed:
+                self._patched = size
+        dev = self._pinned(size).to(device, non_blocking=True)
         self._dev = dev
         views = []
         for arr, off in zip(self._chunks, self._offsets):
@@ -1290,9 +1298,9 @@ class GhostPlan:
         pack = _Pack()
         idx = {}
         seg_st, seg_ln, seg_ex = reg.arrays()
-        idx["seg_start"] = pack.add(seg_st)
-        idx["seg_len"] = pack.add(seg_ln)
-        idx["seg_ex"] = pack.add(seg_ex)
+        idx["seg_start"] = pack.add(seg_st, fixed=True)
+        idx["seg_len"] = pack.add(seg_ln, fixed=True)
+        idx["seg_ex"] = pack.add(seg_ex, fixed=True)
         self._launch: list[tuple] = []
         tabs = [("pack", None, pft), ("planes", None, pl)]
         for key in sorted(pj, key=lambda k: (str(k[0]), k[1])):
@@ -1318,13 +1326,13 @@ class GhostPlan:
         tab_idx = []
         for name, dt, t in tabs:
             probs, ws, total = t.arrays()
-            tab_idx.append((name, dt, pack.add(probs), pack.add(ws), len(t.rows), total,
+            tab_idx.append((name, dt, pack.add(probs), pack.add(ws, fixed=True), len(t.rows), total,
                             (t.nbytes, t.nflops, t.io_bytes)))
-        idx["gstart"] = pack.add(gstart)
+        idx["gstart"] = pack.add(gstart, fixed=True)
         idx["thr"] = pack.add(np.asarray(self.clip.thresholds, dtype=np.float64))
         guards = self.clip.guards or [(1.0, 0.0, torch.float32)]
         idx["guard"] = pack.add(np.asarray([[g[0], g[1]] for g in guards], dtype=np.float64).reshape(-1))
-        idx["cls_dt"] = pack.add(np.asarray([dtype_code(g[2]) for g in guards], dtype=np.int32))
+        idx["cls_dt"] = pack.add(np.asarray([dtype_code(g[2]) for g in guards], dtype=np.int32), fixed=True)
         views = pack.upload(dev)
         self._views = views
         self._pack = pack

@@ -20,7 +20,7 @@ from opaque_amd import _native as N
 from opaque_amd import capture
 from opaque_amd.clipping import auto_clipped_grad, clipped_grad
 from opaque_amd.engine import (LORA_PTRS, ClipSpec, GhostPlan, LeafOut, LinearSite, LoraSite, MaterializedLeaf,
-                               Segments, plan_key)
+                               Segments, _Pack, plan_key)
 from opaque_amd.guard import guard_constants, leaf_guards
 
 pytestmark = pytest.mark.gpu
@@ -215,3 +215,30 @@ def test_drop_in_reuses_its_plan():
         assert torch.equal(a.pytree[k], snap[k]), k
     assert torch.equal(aux_a.grad_norms, norms_a)
     print(f"drop-in calls after the first: {[round(t * 1e3, 2) for t in times]} ms", flush=True)
+
+
+def test_rebind_uploads_only_the_tables_it_patches(monkeypatch):
+    """Segment arrays, work starts and launch maps (two words for every workgroup of the streamed factor pass) never
+    change: a rebind copies the problem tables, thresholds and guards, each on a 256-byte boundary."""
+    print("rebind: bytes uploaded", flush=True)
+    leaves, clip = _spec([0.5, 0.8])
+    n_ex = 1024
+    seg = Segments.padded(n_ex, 8)
+    l1, n1, m1 = _inputs(1, n_ex=n_ex, T=8, products=True)
+    kw = dict(segments=seg, leaves=leaves, device=DEV)
+    plan = GhostPlan(clip=clip, lora_sites=l1, linear_sites=n1, materialized=m1, **kw)
+    l2, n2, m2 = _inputs(2, n_ex=n_ex, T=8, products=True)
+    sizes, pinned = [], _Pack._pinned
+
+    def record(self, *args):
+        sizes.append(pinned(self, *args).numel())
+        return pinned(self, *args)
+
+    monkeypatch.setattr(_Pack, "_pinned", record)
+    assert plan.rebind(l2, m2, n2, clip)
+    tables = sum((t[2].numel() * 8 + 255) // 256 * 256 for t in plan.tables)
+    assert len(sizes) == 1 and sizes[0] <= tables + 2 * 256, (sizes, tables)
+    got = _snapshot(plan.run())
+    want = _snapshot(GhostPlan(clip=clip, lora_sites=l2, linear_sites=n2, materialized=m2, **kw).run())
+    torch.cuda.synchronize()
+    _same(got, want)
