@@ -102,7 +102,7 @@ def kernel_label(stage, key):
         return {"sqnorm": "k_sqnorm", "scale_sum": "k_scale_sum", "nonfinite": "k_nonfinite_cols",
                 "pack": "k_pack_factors", "planes": "k_pack_planes",
                 "factor_project": "k_factor_project_bf16"}[stage]
-    if stage in ("factor_stream", "factor_stream_long"):
+    if stage == "factor_stream":
         # One launch over the tables of several rank block counts; one table alone names its count.
         return "k_factor_stream_bf16" if isinstance(key, tuple) else f"k_factor_stream_bf16<{key}>"
     dt, nkb = key

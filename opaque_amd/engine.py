@@ -546,9 +546,6 @@ def plan_key(*, segments: Segments, leaves: list[LeafOut], clip: ClipSpec, lora_
 # ---------------------------------------------------------------------------
 
 
-# The streamed factor pass: the tables of such a stage (one per rank block
-# count) go out in one launch.
-_STREAM_STAGES = ("factor_stream", "factor_stream_long")
 # Workgroups of the streamed pass a CU holds (two stages of 40 KB each), and
 # how many times over the chip's slots should be filled: below that, segments
 # are split into smaller column groups than odp_seg_factor_stream_groups()'s.
@@ -1064,12 +1061,6 @@ class GhostPlan:
         for _, _, row, blocks, nbytes, io, fl in sorted(fused_rows, key=lambda t: (t[0], t[1])):
             fp.add(row, blocks, nbytes, fl, io=io)
         fst = self._stream_tables(stream_rows)
-        # Plans whose segments all fit odp_factor_project_max_len() rows, and
-        # the others, run the same launch (odp_seg_factor_stream_tables) as
-        # different stages.
-        limit = int(lib.odp_factor_project_max_len())
-        longest = max((t[2].max_len for rows in stream_rows.values() for t in rows), default=0)
-        stream_stage = "factor_stream" if longest <= limit else "factor_stream_long"
 
         sq = _Table(N.SQ_FIELDS)
         mat_pe: dict[int, torch.Tensor] = {}
@@ -1307,7 +1298,7 @@ class GhostPlan:
             tabs.append(("project", key, pj[key]))
         tabs.append(("factor_project", None, fp))
         for nkb in sorted(fst):
-            tabs.append((stream_stage, nkb, fst[nkb]))
+            tabs.append(("factor_stream", nkb, fst[nkb]))
         for key in sorted(ft, key=lambda k: (str(k[0]), k[1])):
             tabs.append(("factor", key, ft[key]))
         tabs.append(("sqnorm", None, sq))
@@ -1346,7 +1337,7 @@ class GhostPlan:
         self.seg_start, self.seg_len, self.seg_ex = (views[idx[k]] for k in ("seg_start", "seg_len", "seg_ex"))
         self.gstart, self.thr = views[idx["gstart"]], views[idx["thr"]]
         self.guard, self.cls_dt = views[idx["guard"]], views[idx["cls_dt"]]
-        self._stream_arg_cache: dict[str, tuple] = {}
+        self._stream_arg_cache: tuple | None = None
         self.tables = [(name, dt, views[pi], views[wi], n, total) for name, dt, pi, wi, n, total, _ in tab_idx]
         # Per launch, in launch order: (stage, key, workgroups, algorithmic bytes, algorithmic flops,
         # contract bytes: the part of the bytes that reads activations and
@@ -1355,7 +1346,7 @@ class GhostPlan:
         for name, dt, _, _, _, total, nb in tab_idx:
             if total <= 0:
                 continue
-            if info and name in _STREAM_STAGES and info[-1][0] == name:  # one launch takes them all
+            if info and name == "factor_stream" == info[-1][0]:  # one launch takes the tables of every rank block count
                 prev = info.pop()
                 keys = (prev[1] if isinstance(prev[1], tuple) else (prev[1],)) + (dt,)
                 info.append((name, keys, prev[2] + total, *(a + b for a, b in zip(prev[3:], nb))))
@@ -1882,13 +1873,13 @@ class GhostPlan:
         """The per-example factor gradients each LoRA leaf stored ([n_seg * r * M], parameter dtype)."""
         return [self.pe[dt][o : o + n] for dt, o, n in self._pe_slices]
 
-    def _stream_args(self, stage: str) -> tuple:
-        """Host arrays of the stage's tables for odp_seg_factor_stream_tables."""
-        args = self._stream_arg_cache.get(stage)
+    def _stream_args(self) -> tuple:
+        """Host arrays of the streamed tables for odp_seg_factor_stream_tables."""
+        args = self._stream_arg_cache
         if args is None:
-            by_nkb = {t[1]: t for t in self.tables if t[0] == stage and t[5] > 0}
+            by_nkb = {t[1]: t for t in self.tables if t[0] == "factor_stream" and t[5] > 0}
             rows = [by_nkb.get(k + 1) for k in range(4)]
-            args = self._stream_arg_cache[stage] = (
+            args = self._stream_arg_cache = (
                 (ctypes.c_void_p * 4)(*[t[2].data_ptr() if t else None for t in rows]),
                 (ctypes.c_void_p * 4)(*[t[3].data_ptr() if t else None for t in rows]),
                 (ctypes.c_int32 * 4)(*[t[4] if t else 0 for t in rows]),
@@ -1899,7 +1890,7 @@ class GhostPlan:
     def run(self, events: dict | None = None, launch_log: list | None = None) -> GhostResult:
         """Launch the step on the current stream.
 
-        ``events`` may map a stage name ("project", "factor_project",
+        ``events`` may map a stage name ("pack", "planes", "project", "factor_project", "factor_stream",
         "factor", "sqnorm", "nonfinite", "lin_norm", "clip", "scale_sum", "lin_sum") to a
         (start, end) pair of torch.cuda.Event that are recorded around that
         stage's launches ("lin_sum" spans the clipped sums of full weights:
@@ -1939,8 +1930,8 @@ class GhostPlan:
                                                    self.seg_start.data_ptr(), self.seg_len.data_ptr(),
                                                    self.seg_ex.data_ptr(), self.part.data_ptr(),
                                                    self.n_slots), name)
-            elif name in _STREAM_STAGES:
-                N.check(lib.odp_seg_factor_stream_tables(s, *self._stream_args(name), self.seg_start.data_ptr(),
+            elif name == "factor_stream":
+                N.check(lib.odp_seg_factor_stream_tables(s, *self._stream_args(), self.seg_start.data_ptr(),
                                                          self.seg_len.data_ptr(), self.seg_ex.data_ptr(),
                                                          self.part.data_ptr(), self.n_slots), name)
             elif name == "factor":
@@ -1965,7 +1956,7 @@ class GhostPlan:
         # on MI355X.)
         names = [t[0] for t in live]
         for idx, (name, dt, probs, ws, n, total) in enumerate(live):
-            if name in _STREAM_STAGES and name in names[:idx]:
+            if name == "factor_stream" and name in names[:idx]:
                 continue  # went out with the stage's first table
             if name in ev and name not in names[:idx]:
                 ev[name][0].record(main)
@@ -1973,7 +1964,7 @@ class GhostPlan:
             launch(name, dt, probs, ws, n, total, stream)
             if end_ev is not None:
                 end_ev.record(main)
-            if name in ev and (name in _STREAM_STAGES or name not in names[idx + 1:]):
+            if name in ev and (name == "factor_stream" or name not in names[idx + 1:]):
                 ev[name][1].record(main)
         if "clip" in ev:
             ev["clip"][0].record()

@@ -11,9 +11,9 @@ rows of sites with different scalings, and activations shared by two or
 three sites of rank 16, one of them with a frozen A: a rank block without a
 leaf), the mirrored order of a down projection, sites bringing the seam's V
 and U, widths that split a segment's tiles into several groups with a
-partial last tile, empty, single-row, longest and unaligned segments, and
-the cases that keep the tiled pass (leaves off the 16-row blocks, a segment
-past the length limit).
+partial last tile, empty, single-row and unaligned segments, one past
+odp_factor_project_max_len() rows, and the case that keeps the tiled pass
+(leaves off the 16-row blocks).
 """
 
 from __future__ import annotations
@@ -91,7 +91,7 @@ def _compare(seg, sites, leaves, expect_stream=True, fuse=True):
 CASES = [
     # n_ex, T, lengths, d_in, d_outs, ranks, frozen
     (5, 96, [96, 33, 1, 70, 64], 136, [264], [8], ()),             # partial last tile, length 1
-    (3, 1081, [1081, 0, 517], 64, [512], [16], ()),                # longest segment, empty segment
+    (3, 1081, [1081, 0, 517], 64, [512], [16], ()),                # longest fused segment, empty segment
     (4, 40, [40, 39, 17, 25], 96, [1000, 200], [12, 4], ()),       # two sites on one X: dA stays tiled
     (3, 64, [64, 50, 9], 128, [256, 136], [8, 8], ((0, "B"), (1, "A"))),  # frozen factors
     (4, 80, [80, 33, 1, 64], 520, [136], [16], ()),                # mirrored: d_in > d_out
@@ -130,13 +130,22 @@ def test_unaligned_segments():
     _compare(seg, sites, leaves)
 
 
-def test_segment_past_the_limit_keeps_the_tiled_pass():
+def test_segment_past_the_fused_limit_streams():
+    """The fused G side holds odp_factor_project_max_len() rows; the streamed
+    pass takes a longer segment, as the same stage, which events and
+    launch_log time under its name."""
     limit = int(N.load().odp_factor_project_max_len())
     T = limit + 21
     print(f"factor stream: segment of {T} rows (limit {limit})", flush=True)
     seg = Segments.padded(2, T, [T, 40])
     sites, leaves = _sites(2 * T, 96, [200], [16], seed=7)
-    _compare(seg, sites, leaves, expect_stream=False)
+    on = _compare(seg, sites, leaves, expect_stream=True)
+    ev = {"factor_stream": tuple(torch.cuda.Event(enable_timing=True) for _ in range(2))}
+    log = []
+    on.run(events=ev, launch_log=log)
+    torch.cuda.synchronize()
+    assert ev["factor_stream"][0].elapsed_time(ev["factor_stream"][1]) > 0
+    assert [i[0] for i in on.launch_info] == [e[0] for e in log] and "factor_stream" in [e[0] for e in log]
 
 
 @pytest.mark.parametrize("shared", [False, True])
