@@ -53,6 +53,8 @@ def _f64_bits(x: float) -> int:
 
 # Bytes from one row to the next that 64-token steps address within 32 bits.
 MAX_ROW_PITCH = 1 << 24
+# A launch holds fewer than 2^32 threads, in workgroups of 256.
+MAX_WORKGROUPS = 1 << 24
 
 
 def _rows(t: torch.Tensor) -> torch.Tensor:
@@ -1284,6 +1286,8 @@ class GhostPlan:
                 + rank * M * out.element_size() * (2 if self.out2 is not None else 1),
                 io=rank * M * out.element_size() * (2 if self.out2 is not None else 1),
             )
+        if sum(ss.blocks) >= MAX_WORKGROUPS:  # several tiles a workgroup
+            ss.blocks = [int(lib.odp_scale_sum_blocks(r[N.SS_RANK] * r[N.SS_M])) for r in ss.rows]
 
         # Upload everything in one copy.
         pack = _Pack()

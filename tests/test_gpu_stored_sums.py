@@ -235,3 +235,29 @@ def test_one_long_group_among_short_ones(name):
     assert torch.allclose(scales[0], (thr.view(-1, 1) / want.sqrt()).clamp(max=1.0), rtol=1e-6)
     assert torch.equal(clipped.bool(), gn > thr.float().view(-1, 1))
     assert all(torch.equal(a, b) for a, b in zip(*runs))
+
+
+def test_more_tiles_than_one_launch_holds():
+    """A leaf of 2^32 + 3 bfloat16 values, off the 16-byte grid: one element a thread would be 2^24 workgroups and
+    more, 2^32 threads, which a launch does not hold; the workgroups walk over several tiles instead."""
+    print("stored sums: 2^32 + 3 elements", flush=True)
+    n, q = 2**32 + 3, 2**20 + 7
+    m = n // q
+    base = torch.randn(q, device=DEV, generator=torch.Generator(device=DEV).manual_seed(1)).to(torch.bfloat16)
+    pe = torch.zeros(1, n, device=DEV, dtype=torch.bfloat16)
+    pe[0, : m * q].view(m, q).copy_(base)
+    pe[0, n - 1] = 2.0
+    leaves = [LeafOut((n,), torch.bfloat16)]
+    plan = GhostPlan(segments=Segments.padded(1, 1), leaves=leaves, clip=_clip(leaves, torch.bfloat16, [1e30]),
+                     materialized=[MaterializedLeaf(pe, 0)], device=DEV)
+    assert sum(t[5] for t in plan.tables if t[0] == "scale_sum") < 2**24
+    res = plan.run()
+    torch.cuda.synchronize()
+    norm = (m * base.float().square().double().sum() + 4.0).sqrt()
+    assert torch.allclose(res.norms.double(), norm, rtol=1e-6)
+    want = _sums(base.view(1, q), res.scales[0, 0], torch.bfloat16)[0]
+    got = res.leaves[0]
+    assert bool((got[: m * q].view(m, q) == want).all())
+    rest = torch.zeros(n - m * q, dtype=torch.bfloat16)
+    rest[-1] = 2.0
+    assert torch.equal(got[m * q :], _sums(rest.view(1, -1), res.scales[0, 0], torch.bfloat16)[0])
