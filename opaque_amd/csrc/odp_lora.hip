@@ -1593,30 +1593,42 @@ extern "C" int odp_seg_factor_stream_tables(odp_stream_t stream, const int64_t* 
     odp_set_error("%s: null table arrays", what);
     return ODP_ERR_INVALID_ARGUMENT;
   }
-  FactorTables T = {};
   int64_t blocks = 0;
   for (int k = 0; k < 4; ++k) {
     int rc = odp_check_table(what, problems[k], block_map[k], n_prob[k], total_blocks[k]);
     if (rc != ODP_OK) return rc;
+    blocks += total_blocks[k];
+  }
+  if (blocks == 0) return ODP_OK;
+  if (seg_row_start == nullptr || seg_row_len == nullptr || seg_example == nullptr || part == nullptr ||
+      part_stride <= 0) {
+    odp_set_error("%s: null segment/partial arrays or part_stride <= 0", what);
+    return ODP_ERR_INVALID_ARGUMENT;
+  }
+  // Tables whose workgroups together pass what one launch holds (2^32 threads)
+  // go out in several.
+  constexpr int64_t MAX_BLOCKS = ((int64_t)1 << 24) - 1;
+  FactorTables T = {};
+  blocks = 0;
+  auto launch = [&]() {
+    hipLaunchKernelGGL(k_factor_stream_bf16, dim3((unsigned)blocks), dim3(256), 0, odp_hip_stream(stream), T,
+                       INT32_MAX, seg_row_start, seg_row_len, seg_example, part, part_stride);
+    T = FactorTables{};
+    blocks = 0;
+    return odp_check_launch(what);
+  };
+  for (int k = 3; k >= 0; --k) {  // the kernel's order
+    if (blocks > 0 && blocks + total_blocks[k] > MAX_BLOCKS) {
+      const int rc = launch();
+      if (rc != ODP_OK) return rc;
+    }
     T.probs[k] = problems[k];
     T.map[k] = block_map[k];
     T.n_prob[k] = n_prob[k];
     T.total[k] = total_blocks[k];
     blocks += total_blocks[k];
   }
-  if (blocks == 0) return ODP_OK;
-  if (blocks >= INT32_MAX) {
-    odp_set_error("%s: the tables exceed the int32 workgroup range", what);
-    return ODP_ERR_UNSUPPORTED;
-  }
-  if (seg_row_start == nullptr || seg_row_len == nullptr || seg_example == nullptr || part == nullptr ||
-      part_stride <= 0) {
-    odp_set_error("%s: null segment/partial arrays or part_stride <= 0", what);
-    return ODP_ERR_INVALID_ARGUMENT;
-  }
-  hipLaunchKernelGGL(k_factor_stream_bf16, dim3((unsigned)blocks), dim3(256), 0, odp_hip_stream(stream), T, INT32_MAX,
-                     seg_row_start, seg_row_len, seg_example, part, part_stride);
-  return odp_check_launch(what);
+  return blocks > 0 ? launch() : ODP_OK;
 }
 
 extern "C" int odp_seg_factor(odp_stream_t stream, int dtype, const int64_t* problems,

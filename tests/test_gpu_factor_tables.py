@@ -108,6 +108,107 @@ def test_sites_of_different_scalings_stream_their_own_rows():
     _check("shared_r24", (2.0, 0.5))
 
 
+# Rank blocks: (first column, rank) of each leaf.  A block without a leaf, ranks below and at 16, and for the
+# tables entry leaves that span blocks.
+DIRECT = {1: [(0, 16)], 2: [(0, 9), (16, 16)], 3: [(0, 16), (32, 3)], 4: [(0, 40), (48, 16)]}
+
+
+class _Direct:
+    """One problem of nkb rank blocks for a direct call: segments of one step, none and several, unaligned, below
+    odp_factor_project_max_len() rows; 18 column tiles, the last partial."""
+
+    M, starts, lens = 4360, [0, 61, 61, 129], [61, 0, 67, 700]
+
+    def __init__(self, nkb):
+        g = torch.Generator(device=DEV).manual_seed(nkb)
+        self.nkb, self.leaves, n_rows = nkb, DIRECT[nkb], 840
+        self.r = self.leaves[-1][0] + self.leaves[-1][1]
+        self.ldq = (n_rows + 32 + 7) // 8 * 8
+        self.P = torch.randn(n_rows, self.M, device=DEV, generator=g).to(torch.bfloat16)
+        self.Q = torch.randn(16 * nkb, self.ldq, device=DEV, generator=g).to(torch.bfloat16)
+        self.tiles = int(N.load().odp_seg_factor_tiles(N.DTYPE_BF16, self.M, self.r))
+        self.n_slots = len(self.leaves) * N.FT_WAVE_SLOTS * self.tiles
+        self.seg = [torch.tensor(v, device=DEV, dtype=torch.int32) for v in (self.starts, self.lens, range(4))]
+
+    def outputs(self):
+        pes = [torch.full((4, rk, self.M), 7.0, device=DEV, dtype=torch.bfloat16) for _, rk in self.leaves]
+        return pes, torch.full((4, self.n_slots), -1.0, device=DEV, dtype=torch.float64)
+
+    def row(self, pes, groups=0):
+        row = [0] * N.FT_FIELDS
+        row[N.FT_P], row[N.FT_LDP], row[N.FT_M] = self.P.data_ptr(), self.M, self.M
+        row[N.FT_Q], row[N.FT_LDQ], row[N.FT_R] = self.Q.data_ptr(), self.ldq, self.r
+        row[N.FT_NSEG], row[N.FT_NLEAF], row[N.FT_GROUPS] = 4, len(self.leaves), groups
+        row[N.FT_SCALING] = int(torch.tensor([2.0], dtype=torch.float64).view(torch.int64).item())
+        for k, ((col, rk), pe) in enumerate(zip(self.leaves, pes)):
+            row[N.FT_LEAF0 + 3 * k : N.FT_LEAF0 + 3 * k + 3] = [pe.data_ptr(), col | rk << 16 | 1 << 32,
+                                                                k * N.FT_WAVE_SLOTS * self.tiles]
+        return torch.tensor(row, dtype=torch.int64, device=DEV)
+
+    def args(self, part):
+        return (*(t.data_ptr() for t in self.seg), part.data_ptr(), self.n_slots)
+
+    def tiled(self):
+        pes, part = self.outputs()
+        row, total = self.row(pes), 4 * self.tiles
+        ws = torch.tensor([0, total], device=DEV, dtype=torch.int32)
+        N.check(N.load().odp_seg_factor(torch.cuda.current_stream().cuda_stream, N.DTYPE_BF16, row.data_ptr(),
+                                        ws.data_ptr(), 1, total, *self.args(part), self.nkb), "tiled")
+        torch.cuda.synchronize()
+        assert (part >= 0).all()  # every slot is written
+        return pes, part
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("groups", [1, 5, 18])
+@pytest.mark.parametrize("nkb", [1, 2, 3])
+def test_one_streamed_table_equals_the_tiled_pass(nkb, groups):
+    """odp_seg_factor_stream (no plan launches it): rows and every partial slot, bit for bit."""
+    print(f"streamed factor table: {nkb} rank blocks, {groups} groups", flush=True)
+    d = _Direct(nkb)
+    want, want_part = d.tiled()
+    pes, part = d.outputs()
+    row, total = d.row(pes, groups), 4 * groups
+    ws = torch.tensor([0, total], device=DEV, dtype=torch.int32)
+    N.check(N.load().odp_seg_factor_stream(torch.cuda.current_stream().cuda_stream, row.data_ptr(), ws.data_ptr(), 1,
+                                           total, *d.args(part), nkb), "stream")
+    torch.cuda.synchronize()
+    assert torch.equal(part, want_part)
+    assert all(torch.equal(a, b) for a, b in zip(pes, want))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("spare", [0, 9 << 20])
+def test_streamed_tables_called_directly(spare):
+    """Four tables at once; with spare workgroups (past a row's segments, which have nothing to do) two of them
+    hold 2^23 and more, together more than one launch may have."""
+    print(f"streamed factor tables: four at once, {spare} spare workgroups", flush=True)
+    ds = [_Direct(k + 1) for k in range(4)]
+    wants = [d.tiled() for d in ds]
+    n_slots = max(d.n_slots for d in ds)
+    outs = [d.outputs() for d in ds]
+    # One partials buffer for the call: the tables' examples lie one after the other.
+    part = torch.full((16, n_slots), -1.0, device=DEV, dtype=torch.float64)
+    segs = [torch.cat([d.seg[j] for d in ds]) for j in range(2)] + [torch.arange(16, device=DEV, dtype=torch.int32)]
+    groups, rows, maps = 5, [], []
+    for k, (d, (pes, _)) in enumerate(zip(ds, outs)):
+        row = d.row(pes, groups)
+        row[N.FT_SEG_FIRST] = 4 * k
+        work = torch.stack([torch.zeros(4 * groups, dtype=torch.int32), torch.arange(4 * groups, dtype=torch.int32)], 1)
+        idle = torch.tensor([[0, 4 * groups]], dtype=torch.int32, device=DEV).expand(spare if k in (0, 2) else 0, 2)
+        rows.append(row)
+        maps.append(torch.cat([idle, work.to(DEV)]).contiguous())  # the work last
+    call = N.load().odp_seg_factor_stream_tables
+    N.check(call(torch.cuda.current_stream().cuda_stream, (ctypes.c_void_p * 4)(*[t.data_ptr() for t in rows]),
+                 (ctypes.c_void_p * 4)(*[t.data_ptr() for t in maps]), (ctypes.c_int32 * 4)(1, 1, 1, 1),
+                 (ctypes.c_int32 * 4)(*[t.shape[0] for t in maps]), *(t.data_ptr() for t in segs), part.data_ptr(),
+                 n_slots), "tables")
+    torch.cuda.synchronize()
+    for k, (d, (pes, _), (want, want_part)) in enumerate(zip(ds, outs, wants)):
+        assert torch.equal(part[4 * k : 4 * k + 4, : d.n_slots], want_part), k
+        assert all(torch.equal(a, b) for a, b in zip(pes, want)), k
+
+
 def test_argument_checks():
     lib = N.load()
     null, bad = (ctypes.c_void_p * 4)(), (ctypes.c_void_p * 4)(8, None, None, None)
