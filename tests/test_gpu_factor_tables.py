@@ -58,7 +58,8 @@ def _case(name, scalings=(2.0,)):
         for k, (d_out, r) in enumerate(outs):
             gt, A, B = rnd(n_rows, d_out, scale=0.3), rnd(d_in, r, scale=1 / math.sqrt(d_in)), rnd(r, d_out, scale=0.05)
             n = len(leaves)
-            leaves += [LeafOut((d_in, r), torch.bfloat16), LeafOut((r, d_out), torch.bfloat16)]
+            leaves += [LeafOut((d_in, r), torch.bfloat16, group=n),
+                       LeafOut((r, d_out), torch.bfloat16, group=n + 1)]
             sites.append(LoraSite(x, gt, A, B, scalings[k % len(scalings)], a_leaf=n, b_leaf=n + 1, v=x @ A,
                                   u=gt @ B.t().contiguous()))
     return seg, sites, leaves
@@ -67,16 +68,16 @@ def _case(name, scalings=(2.0,)):
 def _plan(seg, sites, leaves, stream):
     _, rnd = leaf_guards([lf.shape for lf in leaves], [torch.bfloat16] * len(leaves))
     rel, ab = guard_constants(torch.bfloat16, rnd)
-    clip = ClipSpec(mode=N.CLIP_AUTOS, thresholds=[1.0], effective=1.0, gamma=0.01, normalize_by=2.0,
-                    guards=[(rel, ab, torch.bfloat16)])
+    clip = ClipSpec(mode=N.CLIP_AUTOS, thresholds=[1.0] * len(leaves), effective=math.sqrt(len(leaves)), gamma=0.01,
+                    normalize_by=2.0, guards=[(rel, ab, torch.bfloat16)])
     return GhostPlan(segments=seg, leaves=leaves, clip=clip, lora_sites=sites, device=DEV, stream_factors=stream)
 
 
 def _outputs(plan):
     res = plan.run()
     torch.cuda.synchronize()
-    return [t.clone() for t in plan.pe_views()] + [t.clone() for t in res.leaves] + [res.norms.clone(),
-                                                                                   plan.part.sum(1)]
+    return [t.clone() for t in plan.pe_views()] + [t.clone() for t in res.leaves] + [
+        res.norms.clone(), res.group_norms.clone(), plan.part.clone()]
 
 
 def _check(name, scalings=(2.0,)):
@@ -87,8 +88,13 @@ def _check(name, scalings=(2.0,)):
     assert "factor_stream" in stages and ("factor" in stages) == name.endswith("tiled"), stages
     for k, (a, b) in enumerate(zip(_outputs(on), _outputs(off))):
         assert torch.isfinite(a.float()).all(), k
-        # The partial slots are summed here in another order than the slots'.
-        assert torch.equal(a, b) if a.dtype != torch.float64 else torch.allclose(a, b, rtol=1e-13), k
+        assert torch.equal(a, b), k
+    # Each leaf's group norm is that of its stored rows: fp64 sums of float32 squares, returned in float32.
+    norms = on.run().group_norms.double()
+    torch.cuda.synchronize()
+    for k, pe in enumerate(on.pe_views()):
+        want = pe.view(seg.n_ex, -1).float().square().double().sum(1).sqrt()
+        assert torch.allclose(norms[k], want, rtol=1e-6), k
     return on
 
 

@@ -64,15 +64,20 @@ def _sums(pe, c, out_dtype, nb=3.0):
 ROWS = [(1, 1), (3, 5), (8, 9), (1001, 17), (1024, 8), (2048, 4), (2052, 3), (8191, 2), (8192, 7), (24580, 13)]
 
 
+@pytest.mark.parametrize("offset", [0, 1])
 @pytest.mark.parametrize("second", [False, True])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("n,n_ex", ROWS)
-def test_materialised_rows(n, n_ex, dtype, second):
-    print(f"stored sums: {n} x {n_ex} {dtype} second={second}", flush=True)
+def test_materialised_rows(n, n_ex, dtype, second, offset):
+    """offset: elements from the allocation's start to the leaf.  One past it no row of a length on the 16-byte grid
+    lies on the grid itself: the sums then walk one element a thread over the tiles of 8 or 4, the norms read a
+    head before each row's pieces."""
+    print(f"stored sums: {n} x {n_ex} {dtype} second={second} offset={offset}", flush=True)
     g = torch.Generator(device=DEV).manual_seed(n + n_ex)
     spread = torch.logspace(-1, 1, n_ex, device=DEV).view(-1, 1)
-    # One element past the allocation's start: rows off the 16-byte grid where the dtype and length allow it.
-    pe = (torch.randn(n_ex * n + 1, device=DEV, generator=g)[1:].view(n_ex, n) * spread).to(dtype)
+    pe = torch.empty(n_ex * n + offset, device=DEV, dtype=dtype)[offset:].view(n_ex, n)
+    pe.copy_(torch.randn(n_ex, n, device=DEV, generator=g) * spread)
+    assert (pe.data_ptr() % 16 != 0) == bool(offset)
     pe[0, 0] = float("nan")
     pe[n_ex - 1, n - 1] = float("-inf")
     leaves = [LeafOut((n,), dtype)]
