@@ -230,6 +230,8 @@ int odp_seg_factor_project(odp_stream_t stream, const int64_t* problems,
                            const int32_t* seg_example, double* part, int64_t part_stride);
 
 /* ---- odp_seg_factor_stream: factor rows from given planes, streamed ----
+ * One table found through work_start (odp_seg_factor_stream_tables, which a
+ * GhostPlan launches, takes maps, longer segments and higher ranks).
  * Replaces the same per-sample products as odp_seg_factor
  * (opaque-patches/src/opaque/api/patches/kernels/lora.py:164-176: dB[i] =
  * s (X[i] A)^T G[i] with Q = the V plane, or dA[i]^T = s (G[i] B^T)^T X[i]
@@ -241,8 +243,9 @@ int odp_seg_factor_project(odp_stream_t stream, const int64_t* problems,
  * marked non-temporal.  The row's ODP_FT_GROUPS field splits each
  * segment's 256-column tiles into that many groups of consecutive tiles,
  * one workgroup each (1 <= groups <= tiles; odp_seg_factor_stream_groups(M)
- * is the default): workgroups per problem = n_seg * groups.  Segments may
- * be at most odp_factor_project_max_len() rows long; a longer one that
+ * is the default): workgroups per problem = n_seg * groups.  The row pitch
+ * is at least ODP_FT_M, and a segment's rows span less than 2 GiB.  Segments
+ * may be at most odp_factor_project_max_len() rows long; a longer one that
  * does not fit gets NaN partials and nothing else written.               */
 enum { ODP_FT_GROUPS = 23 };
 int64_t odp_seg_factor_stream_groups(int64_t M);

@@ -184,13 +184,14 @@ __global__ __launch_bounds__(CL_THREADS) void k_clip_factors(
   }
 }
 
-// Clipped sum of one leaf per problem: 8 consecutive elements per thread
-// (one 16-byte load per segment for bf16), summed over the leaf's segments
-// in segment order.  Each term is scale * value rounded to the value's dtype
+// Clipped sum of one leaf per problem, element by element: SS_ELEMS
+// consecutive elements per thread, summed over the leaf's segments in
+// segment order.  Each term is scale * value rounded to the value's dtype
 // (clip_pytree's `scale.to(dtype) * leaf`), accumulated in float32, or in
 // float64 (Acc = double) for float64 values or a float64 compute dtype.
-// This element-wise form serves float64, the float64 sums and raw sums; the
-// form below vectorises float32, bfloat16 and float16.  `raw`: the values
+// This form serves float64, the float64 sums, raw sums and transposed leaves
+// that the form below does not take (rows off the 16-byte grid, rank above
+// SS_THREADS); that one has float32, bfloat16 and float16.  `raw`: the values
 // are already scaled (a caller's scale function): each is summed as it is,
 // with scale 1 and no nan_to_num, as the reference sums a scale function's
 // output (_clipped_fun.py:673-700, 777-782).
@@ -248,7 +249,12 @@ __device__ __forceinline__ void scale_sum_generic(const void* pe, int pdt, int64
 
 // One clipped-sum term: the per-example value with non-finite entries zeroed
 // (nan_to_num), times the scale, rounded to the values' dtype when it is a
-// 16-bit one (scale.to(dtype) * leaf); accumulated in float32.
+// 16-bit one (scale.to(dtype) * leaf); accumulated in float32.  For float32
+// values the compiler contracts product and sum into one fused multiply-add
+// (__fmul_rn and __fadd_rn do not keep it from that), so the product is not
+// rounded by itself as torch and the element-wise form round it: the sums
+// differ from theirs by at most half a unit in the last place a term (1.1e-7
+// of a sum over 64 examples) and lie no further from the float64 sum.
 template <int PDT>
 __device__ __forceinline__ float ss_round(float v) {
   if (PDT == ODP_DTYPE_BF16) return odp_round_bf16(v);
