@@ -264,8 +264,13 @@ class LinearSite:
     index: int | None = None  # slice of a stacked [E, d_out, d_in] leaf (an MoE expert); None: the whole leaf
 
 
-# Time per flop of the Gram-form norm kernel relative to the outer form,
-# measured on MI355X (C4 shapes: 1264 vs 746 TFLOP/s).
+# Time per flop of the Gram-form norm kernel that choose_form assumes,
+# relative to the outer form: the rates on MI355X when the line was drawn were
+# 746 and 1264 TFLOP/s.  The outer kernel without the store has since reached
+# 1360-1416 TFLOP/s at 2048-4096 tokens (4096 x 4096 and 4096 x 14336), 994 at
+# 256, where the Gram form is still the faster by far (64 x 256 tokens, 4096 x
+# 4096: 125 us against 554); on small matrices the two come out even (32 x 400
+# tokens, 768 x 3072: 66 and 69 us).
 GRAM_FLOP_COST = 1.6
 
 # A site in the Gram form whose longest segment spans at least
@@ -276,8 +281,13 @@ GRAM_FLOP_COST = 1.6
 GRAM256_MIN_LEN = 512
 GRAM256_SCRATCH_BYTES = 32 << 30
 GRAM256_ITEM_BYTES = 256 * 256 * 4
-# Its time per flop relative to the outer form, measured on MI355X (C4
-# gate/up/down at 4096 tokens: 1090 vs 1233-1262 TFLOP/s).
+# Its time per flop that choose_form assumes, relative to the outer form (the
+# rates when the line was drawn: 1090 and 1233-1262 TFLOP/s at 4096 tokens).
+# Against the outer kernel's 1360-1416 TFLOP/s it now measures 1.35-1.56 at
+# 3100-4096 tokens, so between about 2048 tokens of 4096 x 4096 (402 us, outer
+# 394) and the line at 3560 the chosen Gram form is up to a quarter slower (8 x
+# 3100: 673 and 602 us; 8 x 3400: 848 and 655); at 512 tokens it is 2.4 times
+# as fast (188 and 456 us).
 GRAM256_FLOP_COST = 1.15
 
 
@@ -551,10 +561,18 @@ def plan_key(*, segments: Segments, leaves: list[LeafOut], clip: ClipSpec, lora_
 # Workgroups of the streamed pass a CU holds (two stages of 40 KB each), and
 # how many times over the chip's slots should be filled: below that, segments
 # are split into smaller column groups than odp_seg_factor_stream_groups()'s.
+# Steps at rank 16 on Llama-shaped layers, with those groups alone and with
+# the slots filled 1, 2, 4 and 8 times: two layers at 4 x 4096 tokens 944, 962,
+# 850, 785 and 795 us, one at 2 x 4096 496 and 255 for the rest (one GPT-2
+# layer at 8 x 512 tokens 72 and 44); four layers at 16 ragged examples of up
+# to 1024 tokens fill the chip by themselves and do not move.
 STREAM_SLOTS_PER_CU = 2
 STREAM_ROUNDS = 4
 STREAM_MIN_ROUNDS = 1
-# Steps (64 tokens of one 256-column tile) a column group should at least hold.
+# Steps (64 tokens of one 256-column tile) a column group should at least hold,
+# so that its fixed cost stays small beside them.  From 1 to 40 of them nothing
+# moved by more than runs differ (two layers at 4 x 4096: 778-793 us), except
+# one layer at 4 x 300 tokens (47.5 us up to 4 steps, 51 from 10).
 STREAM_MIN_STEPS = 10
 
 # Stages launched after the clip factors, in table order.
@@ -792,10 +810,17 @@ class GhostPlan:
         # slot within its leaf (the slices of a stacked leaf follow each other).
         # Sites whose per-example gradients fit in linear_pe_bytes keep them:
         # the outer form stores them (bf16) as it computes the norms, and
-        # the clipped sum becomes a pass over storage.  That beats the Gram
-        # form, which would still need the clipped-sum GEMM, whatever the
-        # sequence length.  The other sites take the faster norm form and
-        # the GEMM.
+        # the clipped sum becomes a pass over storage instead of the GEMM
+        # (with its prescale and column masks) that the norms alone would
+        # still need.  That is the faster of the two on longer sequences
+        # (a Llama-3-8B-shaped layer, 8 examples: 4.00 ms against 4.22 at
+        # 1024 tokens, 6.6 against 9.4 at 2048; eight GPT-2-small layers, 32
+        # examples: 2.06 against 2.59 at 188 tokens on average), where what
+        # each token adds outweighs the fixed bytes per example, and the
+        # slower below (the first at 768 tokens: 3.42 against 3.27, at 256:
+        # 2.26 against 1.57; the second at 122: 1.90 against 1.71, at 43:
+        # 1.71 against 1.06).  linear_pe_bytes=0 asks for the other.  The
+        # sites that do not fit take the faster norm form and the GEMM.
         # One reading of the device memory available to the plan (free plus
         # what torch's allocator holds unused, e.g. an earlier plan's
         # buffers, so repeated calls see the same budgets) is shared by the
