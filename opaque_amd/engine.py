@@ -55,6 +55,10 @@ def _f64_bits(x: float) -> int:
 MAX_ROW_PITCH = 1 << 24
 # A launch holds fewer than 2^32 threads, in workgroups of 256.
 MAX_WORKGROUPS = 1 << 24
+# Segments up to which the clipped sum of a row leaf, of at least SUM_FEW_MIN
+# elements (1024 workgroups), takes 16 elements a thread.
+SUM_FEW_SEGMENTS = 4
+SUM_FEW_MIN = 1 << 22
 
 
 def _rows(t: torch.Tensor) -> torch.Tensor:
@@ -1282,7 +1286,7 @@ class GhostPlan:
                      | (N.DTYPE_BF16 << 56))
             ss.add({N.SS_PE: self.lin_pe[off:].data_ptr(), N.SS_M: M, N.SS_RANK: 1, N.SS_SEG_FIRST: v.first,
                     N.SS_NSEG: v.n_seg, N.SS_OUT: out.data_ptr(), N.SS_FLAGS: flags, N.SS_OUT2: out2},
-                   lib.odp_scale_sum_blocks(M),
+                   self._sum_blocks(M, N.DTYPE_BF16, v.n_seg, not self.sum_f64),
                    v.n_seg * M * 2 + M * out.element_size() * (2 if self.out2 is not None else 1),
                    io=M * out.element_size() * (2 if self.out2 is not None else 1))
         for i, lf in enumerate(self.leaves):
@@ -1306,7 +1310,8 @@ class GhostPlan:
                     N.SS_PE: pe_a, N.SS_M: M, N.SS_RANK: rank, N.SS_SEG_FIRST: v.first,
                     N.SS_NSEG: n_seg, N.SS_OUT: out.data_ptr(), N.SS_FLAGS: flags, N.SS_OUT2: out2,
                 },
-                lib.odp_scale_sum_blocks(rank * M) * self._sum_split(rank * M, pdt),
+                self._sum_blocks(rank * M, pdt, n_seg,
+                                 not (transpose or self.sum_f64 or (self.raw_values and i in mat_pe))),
                 n_seg * rank * M * (self.pe[pe_dt[i]].element_size() if i not in mat_pe else mat_pe[i].element_size())
                 + rank * M * out.element_size() * (2 if self.out2 is not None else 1),
                 io=rank * M * out.element_size() * (2 if self.out2 is not None else 1),
@@ -1860,12 +1865,17 @@ class GhostPlan:
         return row
 
     @staticmethod
-    def _sum_split(n: int, pdt: int) -> int:
-        """Workgroups per 2048 elements of a clipped sum, one tile each: float32
-        and float64 values take 4 elements a thread, 16-bit ones 8, rows of a
-        length off the 16-byte grid one."""
+    def _sum_blocks(n: int, pdt: int, n_seg: int, rows: bool) -> int:
+        """Workgroups of the clipped sum of a leaf of n elements, one tile each:
+        256 threads of 4 elements for float32 and float64 values, of 8 for
+        16-bit ones, of one for rows of a length off the 16-byte grid, and of
+        16 for large row leaves of few segments (SUM_FEW_SEGMENTS)."""
         vec = 4 if pdt in (N.DTYPE_F32, N.DTYPE_F64) else 8
-        return 8 // vec if n % vec == 0 else 8
+        if n % vec:
+            vec = 1
+        elif rows and n_seg <= SUM_FEW_SEGMENTS and n >= SUM_FEW_MIN and pdt != N.DTYPE_F64:
+            vec = 16
+        return (n + 256 * vec - 1) // (256 * vec)
 
     def _leaf_transposed(self, i: int, sites: list[LoraSite]) -> bool:
         # pe rows are [r][M]; A leaves [d_in, r] need the transpose, B leaves [r, d_out] do not.

@@ -95,6 +95,17 @@ def test_materialised_rows(n, n_ex, dtype, second, offset):
         assert _close(res.second_moment[0], want[1], pe, res.scales[0, 0], 2)
 
 
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("dtype,second", [(torch.float32, False), (torch.float32, True), (torch.bfloat16, True),
+                                          (torch.float16, False)])
+@pytest.mark.parametrize("n,n_ex", [(1 << 22, 1), ((1 << 22) + 8, 2), ((1 << 22) + 2056, 3), ((1 << 22) + 4104, 4),
+                                    ((1 << 22) + 8, 5)])
+def test_few_examples_of_large_rows(n, n_ex, dtype, second, offset):
+    """Up to four examples of rows this long take several pieces a thread: whole and partial last workgroups, an odd
+    example, and rows off the grid and five examples, which keep one piece."""
+    test_materialised_rows(n, n_ex, dtype, second, offset)
+
+
 @pytest.mark.parametrize("second", [False, True])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("r", [1, 4, 8, 12, 20, 64])
