@@ -102,14 +102,12 @@ def kernel_label(stage, key):
         return {"sqnorm": "k_sqnorm", "scale_sum": "k_scale_sum", "nonfinite": "k_nonfinite_cols",
                 "pack": "k_pack_factors", "planes": "k_pack_planes",
                 "factor_project": "k_factor_project_bf16"}[stage]
-    if stage == "factor_stream":
-        # One launch over the tables of several rank block counts; one table alone names its count.
-        return "k_factor_stream_bf16" if isinstance(key, tuple) else f"k_factor_stream_bf16<{key}>"
+    if stage == "factor_stream":  # one kernel for the tables of every rank block count
+        return "k_factor_stream_bf16"
     dt, nkb = key
-    base = {"project": "k_project_stream", "factor": "k_factor"}[stage]
-    if dt == torch.bfloat16:
-        return f"{base}_bf16<{nkb}>"
-    return f"{base.replace('_stream', '')}_f32"
+    if stage == "project":
+        return f"k_project_stream_bf16<{nkb}>" if dt == torch.bfloat16 else "k_project_f32"
+    return f"k_factor_{'bf16' if dt == torch.bfloat16 else 'f32'}<{nkb}>"
 
 
 def committed_traffic(label, design_bytes):

@@ -25,12 +25,12 @@ def test_more_than_one_gpu_is_refused():
 
 
 def test_kernel_labels_are_the_device_symbols():
-    assert bench.kernel_label("factor_stream", 1) == "k_factor_stream_bf16<1>"
-    assert bench.kernel_label("factor_stream", 3) == "k_factor_stream_bf16<3>"
+    assert bench.kernel_label("factor_stream", 1) == "k_factor_stream_bf16"
+    assert bench.kernel_label("factor_stream", (1, 2, 3)) == "k_factor_stream_bf16"  # C3's tables, one launch
     assert bench.kernel_label("project", (torch.bfloat16, 2)) == "k_project_stream_bf16<2>"
     assert bench.kernel_label("project", (torch.float32, 1)) == "k_project_f32"
     assert bench.kernel_label("factor", (torch.bfloat16, 3)) == "k_factor_bf16<3>"
-    assert bench.kernel_label("factor", (torch.float32, 1)) == "k_factor_f32"
+    assert bench.kernel_label("factor", (torch.float32, 1)) == "k_factor_f32<1>"
     assert bench.kernel_label("factor_project", None) == "k_factor_project_bf16"
     assert bench.kernel_label("planes", None) == "k_pack_planes"
     assert bench.kernel_label("scale_sum", None) == "k_scale_sum"
@@ -43,7 +43,7 @@ def test_kernel_labels_are_the_device_symbols():
 
 def test_committed_traffic_matches_on_design_bytes_only():
     data = json.loads((ROOT / "profiles" / "traffic.json").read_text())
-    label = "k_factor_stream_bf16<1>"
+    label = bench.kernel_label("factor_stream", (1, 2, 3))
     entry = data["kernels"][label]
     assert bench.committed_traffic(label, entry["algorithmic_bytes"]) == entry["traffic_bytes"]
     assert bench.committed_traffic(label, entry["algorithmic_bytes"] + 1) is None
