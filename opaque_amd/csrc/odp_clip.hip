@@ -35,6 +35,21 @@ __device__ __forceinline__ double finalize_scale(double ratio, double rel, doubl
   return (double)odp_round_to((float)s, dtype);
 }
 
+// Waves per group: 16 for one group, halved until the groups fit side by side
+// (one wave each beyond 8 groups, in rounds of 16 groups).
+__host__ __device__ inline int clip_waves(int n_groups) {
+  int wpg = CL_THREADS / 64;
+  while (wpg > 1 && wpg * n_groups > CL_THREADS / 64) wpg >>= 1;
+  return wpg;
+}
+// Whether a call may have a group too long for its waves.  Four waves come
+// close to what the CU can have in flight, so a group on four or more needs no
+// help.
+inline bool clip_long(int64_t n_slots, int n_groups) {
+  const int wpg = clip_waves(n_groups);
+  return wpg < 4 && n_slots > (int64_t)CL_LONG * wpg;
+}
+
 // One workgroup per example.  Group g owns slots [gstart[g], gstart[g+1]).
 // The sum of an example's partials (a few hundred KB on Llama-shaped
 // models) is bound by what one CU can have in flight, so each thread issues
@@ -50,10 +65,12 @@ __device__ __forceinline__ double finalize_scale(double ratio, double rel, doubl
 // rest: past CL_LONG partials a wave (below, a round of all the waves costs
 // what it saves) and four times its waves' even share (one of 40960 among
 // 16: 17 -> 9 us, of 200000: 67 -> 18; 16 of 8192 each stay side by side, 11 us
-// against 23).
+// against 23).  LONG: the call has slots enough for such a group on waves few
+// enough (clip_long); looking for one costs a call 0.4 us.
 // `status` (optional): a word that k_sqnorm sets when it dropped a write
 // outside the partials; every example then gets a NaN norm, zero scales and
 // clear masks, since the partials are incomplete.
+template <bool LONG>
 __global__ __launch_bounds__(CL_THREADS) void k_clip_factors(
     const double* __restrict__ part, int64_t n_slots, int n_ex, const int64_t* __restrict__ gstart, int n_groups,
     const double* __restrict__ thr, double eff_thr, int mode, double gamma, int n_cls,
@@ -87,8 +104,8 @@ __global__ __launch_bounds__(CL_THREADS) void k_clip_factors(
   if (t < 2 * n_cls) sguard[t] = guard[t];
   if (t < n_cls) scls[t] = cls_dtype[t];
 
-  // This wave's part of the sum of slots [lo, hi), taken by nth threads of
-  // which this is the tg-th (the same in every lane).
+  // This thread's part of the sum of slots [lo, hi), taken by nth threads of
+  // which it is the tg-th.
   auto sum_slots = [&](int64_t lo, int64_t hi, int tg, int nth) __attribute__((always_inline)) {
     double a[CL_DEPTH];
 #pragma unroll
@@ -119,25 +136,24 @@ __global__ __launch_bounds__(CL_THREADS) void k_clip_factors(
     for (int w = CL_DEPTH / 2; w > 0; w >>= 1)
 #pragma unroll
       for (int q = 0; q < w; ++q) a[q] = a[2 * q] + a[2 * q + 1];
-    return rows_sum4(row_sum16(a[0]));
+    return a[0];
   };
-  // Waves per group: 16 for one group, halved until the groups fit side by
-  // side (one wave each beyond 8 groups, in rounds of 16 groups).
   constexpr int NWAVE = CL_THREADS / 64;
-  int wpg = NWAVE;
-  while (wpg > 1 && wpg * n_groups > NWAVE) wpg >>= 1;
-  // Four waves come close to what the CU can have in flight, so a group on
-  // four or more needs no help.
-  const bool few = wpg < 4;
-  const int64_t all = few ? gstart[n_groups] - gstart[0] : 0;
-  auto is_long = [&](int64_t n) { return few && n > (int64_t)CL_LONG * wpg && 4 * n > wpg * all; };
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), nth = 64 * wpg, tg = t & (nth - 1);
-  if (few && t < NWAVE) slong[t] = 0;
+  const int wpg = clip_waves(n_groups);
+  const int64_t all = LONG ? gstart[n_groups] - gstart[0] : 0;
+  auto is_long = [&](int64_t n) { return LONG && n > (int64_t)CL_LONG * wpg && 4 * n > wpg * all; };
+  const int wave = t >> 6, nth = 64 * wpg, tg = t & (nth - 1);
+  if (LONG && t < NWAVE) slong[t] = 0;
   for (int g0 = 0; g0 < n_groups; g0 += NWAVE / wpg) {
     const int g = g0 + wave / wpg;
-    const int64_t lo = g < n_groups ? gstart[g] : 0, hi = g < n_groups ? gstart[g + 1] : 0;
-    const bool longer = is_long(hi - lo);
-    const double ws = sum_slots(lo, longer ? lo : hi, tg, nth);
+    double part_sum = 0.0;
+    bool longer = false;
+    if (g < n_groups) {
+      const int64_t lo = gstart[g], hi = gstart[g + 1];
+      longer = is_long(hi - lo);
+      if (!longer) part_sum = sum_slots(lo, hi, tg, nth);
+    }
+    const double ws = rows_sum4(row_sum16(part_sum));
     if ((t & 63) == 0) red[wave] = ws;
     __syncthreads();
     if (g < n_groups && tg == 0) {
@@ -148,11 +164,11 @@ __global__ __launch_bounds__(CL_THREADS) void k_clip_factors(
     }
     __syncthreads();
   }
-  if (few && __builtin_amdgcn_ballot_w64(slong[t & (NWAVE - 1)] != 0) != 0) {
+  if (LONG && __builtin_amdgcn_ballot_w64(slong[t & (NWAVE - 1)] != 0) != 0) {
     for (int g = 0; g < n_groups; ++g) {
       const int64_t lo = gstart[g], hi = gstart[g + 1];
       if (!is_long(hi - lo)) continue;  // the same for every thread
-      const double ws = sum_slots(lo, hi, t, CL_THREADS);
+      const double ws = rows_sum4(row_sum16(sum_slots(lo, hi, t, CL_THREADS)));
       if ((t & 63) == 0) red[wave] = ws;
       __syncthreads();
       if (t == 0) {
@@ -183,6 +199,10 @@ __global__ __launch_bounds__(CL_THREADS) void k_clip_factors(
       scale_out[((int64_t)k * n_groups + g) * n_ex + ex] =
           finalize_scale(ratio, sguard[2 * k], sguard[2 * k + 1], mode == ODP_CLIP_FIXED, scls[k]);
   }
+}
+
+auto clip_kernel(int64_t n_slots, int n_groups) {
+  return clip_long(n_slots, n_groups) ? k_clip_factors<true> : k_clip_factors<false>;
 }
 
 // Clipped sum of one leaf per problem, element by element: SS_ELEMS
@@ -476,7 +496,7 @@ __device__ __forceinline__ void scale_sum_fast(const void* pe, int64_t M, int ra
 // of as many consecutive tiles, two segments at a time.  The sums are
 // scale_sum_fast's, bit for bit (the same terms in the same order).  2^26
 // values in float32, one example: 157 -> 83 us (6.4 TB/s), two: 176 -> 124;
-// bfloat16: 100 -> 72 and 104 -> 76.
+// bfloat16: 100 -> 75 and 104 -> 80.
 template <bool SECOND, int PDT>
 __device__ __forceinline__ void scale_sum_few(const void* pe, int64_t E, int b, int nblk, int n_seg, int seg_first,
                                               const int32_t* __restrict__ sex, const double* __restrict__ sc,
@@ -521,19 +541,26 @@ __device__ __forceinline__ void scale_sum_few(const void* pe, int64_t E, int b, 
     int s = 0;
     for (; s + 2 <= n_seg; s += 2) group(s, std::integral_constant<int, 2>{});
     if (s < n_seg) group(s, std::integral_constant<int, 1>{});
-#pragma unroll
-    for (int k = 0; k < NT; ++k) {
-      const int64_t e = e0 + k * TILE;
-      if (e >= E) break;
+    // One piece's finish in a loop, the pieces moved down: unrolled, the six
+    // forms' finishes were half of the kernel's code.
+#pragma unroll 1
+    for (int64_t e = e0; e < E && e < e0 + NT * TILE; e += TILE) {
       float x[V];
 #pragma unroll
-      for (int i = 0; i < V; ++i) x[i] = ss_finish(acc[k][i], normalize_by, odt);
+      for (int i = 0; i < V; ++i) x[i] = ss_finish(acc[0][i], normalize_by, odt);
       ss_put<V>(out, e, odt, (((uintptr_t)out + e * oes) & (V * oes - 1) & 15) == 0, x);
       if (SECOND) {
 #pragma unroll
-        for (int i = 0; i < V; ++i) x[i] = ss_finish(acc2[k][i], normalize_by, odt);
+        for (int i = 0; i < V; ++i) x[i] = ss_finish(acc2[0][i], normalize_by, odt);
         ss_put<V>(out2, e, odt, (((uintptr_t)out2 + e * oes) & (V * oes - 1) & 15) == 0, x);
       }
+#pragma unroll
+      for (int k = 0; k + 1 < NT; ++k)
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+          acc[k][i] = acc[k + 1][i];
+          if (SECOND) acc2[k][i] = acc2[k + 1][i];
+        }
     }
   }
 }
@@ -582,12 +609,12 @@ __global__ __launch_bounds__(SS_THREADS) void k_scale_sum(
     return;
   }
   const bool rows16 = aligned && E % vec == 0;
-  const bool few = rows16 && !transpose && n_seg <= SS_FEW && (int64_t)nblk * SS_THREADS * vec < E;
+  const bool few = n_seg <= SS_FEW && rows16 && !transpose && (int64_t)nblk * SS_THREADS * vec < E;
 #define ODP_SS_RUN(SECOND, PDT)                                                                                  \
   do {                                                                                                           \
-    if (few)                                                                                                     \
+    if (__builtin_expect(few, 0))                                                                                \
       scale_sum_few<SECOND, PDT>(pe, E, b, nblk, n_seg, seg_first, sex, sc, normalize_by, out, out2, odt);       \
-    else if (transpose || rows16)                                                                                   \
+    else if (transpose || rows16)                                                                                \
       scale_sum_fast<SECOND, PDT, true>(pe, M, rank, transpose != 0, b, nblk, n_seg, seg_first, sex, sc,         \
                                         normalize_by, out, out2, odt, tile);                               \
     else                                                                                                         \
@@ -775,7 +802,7 @@ extern "C" int odp_clip_factors(odp_stream_t stream, const double* part, int64_t
     odp_set_error("odp_clip_factors: null required pointer");
     return ODP_ERR_INVALID_ARGUMENT;
   }
-  hipLaunchKernelGGL(k_clip_factors, dim3(n_ex), dim3(CL_THREADS), 0, odp_hip_stream(stream), part,
+  hipLaunchKernelGGL(clip_kernel(n_slots, n_groups), dim3(n_ex), dim3(CL_THREADS), 0, odp_hip_stream(stream), part,
                      n_slots, n_ex, group_slot_start, n_groups, thresholds, effective_threshold, mode,
                      gamma, n_cls, guard, cls_dtype, scale_out, norm_out, group_norm_out,
                      clipped_out, clipped_total_out, nullptr);
@@ -909,7 +936,7 @@ extern "C" int odp_clip_materialized_noalloc(
     rc = odp_check_launch(what);
     if (rc != ODP_OK) return rc;
   }
-  hipLaunchKernelGGL(k_clip_factors, dim3(n_ex), dim3(CL_THREADS), 0, s, part, n_slots, n_ex, group_slot_start,
+  hipLaunchKernelGGL(clip_kernel(n_slots, n_groups), dim3(n_ex), dim3(CL_THREADS), 0, s, part, n_slots, n_ex, group_slot_start,
                      n_groups, thresholds, effective_threshold, mode, gamma, n_cls, guard, cls_dtype, scale_out,
                      norm_out, group_norm_out, clipped_out, clipped_total_out, status);
   return odp_check_launch(what);
